@@ -294,8 +294,7 @@ int ma_quantize_values(ma_tensor4 src, int B, int H, int T, int D, int group, vo
  * group / row is where they go, and the remaining keep = old_res + T - move tokens are
  * written to the residual rows 0..keep (in place: its rows move down by `move`).  The
  * residual and the new tokens share one dtype (the quantizers' rule follows it), as the
- * reference's [residual | new.to(compute dtype)] tensor does.  Up to three launches,
- * no temporary. */
+ * reference's [residual | new.to(compute dtype)] tensor does.  One launch, no temporary. */
 int ma_append_packed(ma_tensor4 k_res, ma_tensor4 v_res, int old_res, ma_tensor4 k_new, ma_tensor4 v_new, int B,
                      int H, int T, int D, int move, int keep, void *kq, const int64_t skq[4], void *ks, void *kz,
                      const int64_t sks[3], void *vq, const int64_t svq[4], void *vs, void *vz,

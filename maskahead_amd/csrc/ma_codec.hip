@@ -1,6 +1,8 @@
 // Packed-KV codec kernels: whole-prefix dequant, gather of selected entries, and the
 // 4-bit quantizers of the append path.  All integer/byte work, bit-exact against the
 // reference's torch codec (reference.py:35-268).
+#include <algorithm>
+
 #include "ma_common.h"
 #include "ma_quant.h"
 
@@ -198,21 +200,298 @@ struct TwoSrc {
     int na;
 };
 
-// DT: the dtype, a compile-time constant so that a thread's loads are straight-line code
-// (all of them in flight at once) instead of one branch per element
+// One append (or one quantizer call) in one launch.  kv 0 = keys, 1 = values; a workgroup
+// belongs to one (lane, kv) and is one of
+//   head  the key groups that read `a` (the first gh) and, after a barrier, the residual
+//         rows that replace what they read: in place, so one workgroup does both
+//   bulk  BULK tokens of the groups that read `b` alone
+//   copy  COPY residual rows where nothing that is overwritten is read (na = 0: the rows of
+//         `a` are free; move = 0: its rows stay and `b`'s follow them)
+// What bounds it: a block's append (32 residual + 32 new tokens, 4 lanes of D 128) is one
+// load-to-store latency, 6.4 us; an 8 192-token prompt's is latency and the quantizer's VALU
+// work (about 13 operations a value, 3.4 us of it), 12.3 us for 22 MB.  As three launches --
+// two quantizers with 2-byte loads, and two workgroups a lane copying the residual an
+// element at a time -- they took 28.1 and 34.4 us, 20 us of each the residual's copy.
+constexpr int AP_NT = 256;
+constexpr int BULK = 128;     // tokens of a bulk workgroup: a key group per wave at D = 128
+constexpr int COPY = 64;      // rows of a copy workgroup, and of a head's pass
+
+struct AppendArgs {
+    TwoSrc src[2];
+    uint8_t *q[2];
+    int64_t sq[2][4];
+    _Float16 *s[2], *z[2];
+    int64_t ss[2][3];
+    int H, D, lanes, kv0, nkv;   // kv kinds kv0 .. kv0 + nkv - 1
+    int ntok;                    // tokens quantized
+    int keep, first;             // residual rows [first, keep) written from source rows r + ntok
+    int gh, nhead, nbulk;        // head groups; head (0 or 1) and bulk workgroups per (lane, kv)
+};
+
+// the source rows of one lane
+struct RowSrc {
+    const char *a, *b;
+    int64_t sa, sb;   // bytes per row
+    int na;
+};
+
 template <int DT>
-__device__ __forceinline__ float two_load(const TwoSrc &s, int b, int h, int i, int d) {
-    const bool in_a = i < s.na;
-    const char *base = (const char *)(in_a ? s.a.ptr : s.b.ptr);
-    const int64_t sb = in_a ? s.a.s[0] : s.b.s[0], sh = in_a ? s.a.s[1] : s.b.s[1],
-                  st = in_a ? s.a.s[2] : s.b.s[2];
-    const int r = in_a ? i : i - s.na;
-    return ma_load_f(base, b * sb + h * sh + (int64_t)r * st + d, DT);
+__device__ __forceinline__ RowSrc row_src(const TwoSrc &s, int b, int h) {
+    constexpr int ES = DT == MA_F32 ? 4 : 2;
+    RowSrc r;
+    r.a = (const char *)s.a.ptr + (b * s.a.s[0] + h * s.a.s[1]) * ES;
+    r.b = (const char *)s.b.ptr + (b * s.b.s[0] + h * s.b.s[1]) * ES;
+    r.sa = s.a.s[2] * ES;
+    r.sb = s.b.s[2] * ES;
+    r.na = s.na;
+    return r;
 }
 
+__device__ __forceinline__ const char *src_row(const RowSrc &r, int i) {
+    return i < r.na ? r.a + i * r.sa : r.b + (int64_t)(i - r.na) * r.sb;
+}
+
+// N consecutive elements at p as f32; VEC: p is aligned to N elements
+template <int DT, int N, bool VEC>
+__device__ __forceinline__ void load_n(const char *p, float (&x)[N]) {
+    if constexpr (!VEC) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) x[i] = ma_load_f(p, i, DT);
+    } else if constexpr (DT == MA_F32) {
+        typedef __attribute__((ext_vector_type(N < 4 ? N : 4))) float fv;
+#pragma unroll
+        for (int i = 0; i < N; i += 4) {
+            const fv v = *(const fv *)(p + 4 * i);
+#pragma unroll
+            for (int e = 0; e < (N < 4 ? N : 4); ++e) x[i + e] = v[e];
+        }
+    } else {
+        typedef __attribute__((ext_vector_type(N / 2))) uint32_t uv;
+        uint32_t w[N / 2];
+        if constexpr (N == 2) {
+            w[0] = *(const uint32_t *)p;
+        } else {
+            const uv v = *(const uv *)p;
+#pragma unroll
+            for (int i = 0; i < N / 2; ++i) w[i] = v[i];
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const uint16_t h = (uint16_t)(w[i / 2] >> ((i & 1) * 16));
+            x[i] = DT == MA_BF16 ? ma_bf16_to_f32(h) : ma_f16_to_f32(h);
+        }
+    }
+}
+
+// key groups g0, g0 + step, ... below g1 of one lane: thread c of a group's D / 2 = two
+// channels of its 32 tokens, all loads in flight, no exchange between threads
+template <int DT, bool VEC>
+__device__ __forceinline__ void quant_keys(const AppendArgs &A, const RowSrc &R, int b, int h, int g0, int g1) {
+    const int tpg = A.D / 2;
+    const int d = (threadIdx.x % tpg) * 2;
+    constexpr int ES = DT == MA_F32 ? 4 : 2;
+    for (int g = g0 + threadIdx.x / tpg; g < g1; g += AP_NT / tpg) {
+        float x[KG][2];
+        float lo[2] = {INFINITY, INFINITY}, hi[2] = {-INFINITY, -INFINITY};
+#pragma unroll
+        for (int t = 0; t < KG; ++t) load_n<DT, 2, VEC>(src_row(R, g * KG + t) + d * ES, x[t]);
+#pragma unroll
+        for (int t = 0; t < KG; ++t)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                lo[c] = fminf(lo[c], x[t][c]);
+                hi[c] = fmaxf(hi[c], x[t][c]);
+            }
+        const int64_t so = b * A.ss[0][0] + h * A.ss[0][1] + (int64_t)g * A.ss[0][2] + d;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const QuantGroup qp = quant_params(lo[c], hi[c], DT);
+            uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int t = 0; t < KG; ++t) w[t >> 3] |= quant_code(x[t][c], qp, DT) << ((t & 7) * 4);
+            *(uint4 *)(A.q[0] + b * A.sq[0][0] + h * A.sq[0][1] + (int64_t)g * A.sq[0][2] +
+                       (int64_t)(d + c) * A.sq[0][3]) = uint4{w[0], w[1], w[2], w[3]};
+            A.s[0][so + c] = (_Float16)qp.step;
+            A.z[0][so + c] = (_Float16)qp.lo;
+        }
+    }
+}
+
+// value tokens [t0, t1) of one lane: thread = 8 channels of a token, a group's range from
+// its 4 adjacent threads; VB tokens' loads in flight per thread
+template <int DT, bool VEC>
+__device__ __forceinline__ void quant_values(const AppendArgs &A, const RowSrc &R, int b, int h, int t0, int t1) {
+    constexpr int VB = 4;
+    constexpr int ES = DT == MA_F32 ? 4 : 2;
+    const int tpt = A.D / 8, per = AP_NT / tpt;
+    const int oct = threadIdx.x % tpt, cg = oct / 4;
+    for (int j0 = t0 + threadIdx.x / tpt; j0 < t1; j0 += VB * per) {
+        float x[VB][8];
+#pragma unroll
+        for (int u = 0; u < VB; ++u)   // tokens past the end read the last one and are not written
+            load_n<DT, 8, VEC>(src_row(R, min(j0 + u * per, t1 - 1)) + oct * 8 * ES, x[u]);
+#pragma unroll
+        for (int u = 0; u < VB; ++u) {
+            const int j = j0 + u * per;
+            float lo = x[u][0], hi = x[u][0];
+#pragma unroll
+            for (int c = 1; c < 8; ++c) {
+                lo = fminf(lo, x[u][c]);
+                hi = fmaxf(hi, x[u][c]);
+            }
+            lo = fminf(lo, ma_quad<0xB1>(lo));   // lanes ^ 1, then ^ 2
+            lo = fminf(lo, ma_quad<0x4E>(lo));
+            hi = fmaxf(hi, ma_quad<0xB1>(hi));
+            hi = fmaxf(hi, ma_quad<0x4E>(hi));
+            const QuantGroup qp = quant_params(fminf(INFINITY, lo), fmaxf(-INFINITY, hi), DT);
+            uint32_t w = 0;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) w |= quant_code(x[u][c], qp, DT) << (c * 4);
+            if (j < t1) {
+                *(uint32_t *)(A.q[1] + b * A.sq[1][0] + h * A.sq[1][1] + (int64_t)j * A.sq[1][2] +
+                              (int64_t)cg * A.sq[1][3] + (oct % 4) * 4) = w;
+                const int64_t so = b * A.ss[1][0] + h * A.ss[1][1] + (int64_t)j * A.ss[1][2] + cg;
+                if (oct % 4 == 0) A.s[1][so] = (_Float16)qp.step;
+                if (oct % 4 == 1) A.z[1][so] = (_Float16)qp.lo;
+            }
+        }
+    }
+}
+
+// A pass of at most COPY residual rows, from r0: the loads, then (after whatever must come
+// between) the stores.  A thread holds 8 elements of a row.
+template <int DT, bool VEC>
+struct ResidualPass {
+    static constexpr int ES = DT == MA_F32 ? 4 : 2, NW = 2 * ES;
+    static constexpr int MAXR = COPY * 256 / 8 / AP_NT;   // rows per thread at the largest D (256)
+    uint32_t w[MAXR][NW];
+
+    __device__ __forceinline__ void load(const AppendArgs &A, const RowSrc &R, int r0) {
+        const int tpt = A.D / 8, per = AP_NT / tpt, oct = threadIdx.x % tpt, rt = threadIdx.x / tpt;
+#pragma unroll
+        for (int e = 0; e < MAXR; ++e) {
+            const int r = r0 + rt + e * per;
+            if (e * per < COPY && r < A.keep) {
+                const char *p = src_row(R, r + A.ntok) + oct * 8 * ES;
+                if constexpr (VEC) {
+#pragma unroll
+                    for (int i = 0; i < NW; i += 4) {
+                        const uint4 v = *(const uint4 *)(p + 4 * i);
+                        w[e][i] = v.x;
+                        w[e][i + 1] = v.y;
+                        w[e][i + 2] = v.z;
+                        w[e][i + 3] = v.w;
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < NW; ++i)
+                        w[e][i] = ES == 4 ? *(const uint32_t *)(p + 4 * i)
+                                          : (uint32_t) * (const uint16_t *)(p + 4 * i) |
+                                                ((uint32_t) * (const uint16_t *)(p + 4 * i + 2) << 16);
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ void store(const AppendArgs &A, const RowSrc &R, int r0) {
+        const int tpt = A.D / 8, per = AP_NT / tpt, oct = threadIdx.x % tpt, rt = threadIdx.x / tpt;
+#pragma unroll
+        for (int e = 0; e < MAXR; ++e) {
+            const int r = r0 + rt + e * per;
+            if (e * per < COPY && r < A.keep) {
+                char *p = (char *)R.a + r * R.sa + oct * 8 * ES;
+                if constexpr (VEC) {
+#pragma unroll
+                    for (int i = 0; i < NW; i += 4)
+                        *(uint4 *)(p + 4 * i) = uint4{w[e][i], w[e][i + 1], w[e][i + 2], w[e][i + 3]};
+                } else {
+#pragma unroll
+                    for (int i = 0; i < NW; ++i) {
+                        if constexpr (ES == 4) {
+                            *(uint32_t *)(p + 4 * i) = w[e][i];
+                        } else {
+                            *(uint16_t *)(p + 4 * i) = (uint16_t)w[e][i];
+                            *(uint16_t *)(p + 4 * i + 2) = (uint16_t)(w[e][i] >> 16);
+                        }
+                    }
+                }
+            }
+        }
+    }
+};
+
+template <int DT, bool VEC>
+__global__ void __launch_bounds__(AP_NT) append_packed_kernel(AppendArgs A) {
+    const int units = A.lanes * A.nkv;
+    const int u = blockIdx.x / units, y = blockIdx.x % units;
+    const int kv = A.kv0 + y / A.lanes, bh = y % A.lanes, b = bh / A.H, h = bh % A.H;
+    const RowSrc R = row_src<DT>(A.src[kv], b, h);
+    ResidualPass<DT, VEC> pass;
+    if (u < A.nhead) {
+        // the residual's first rows are on their way while the groups are quantized; nothing
+        // is stored to `a` before every thread has read what it needs of it
+        pass.load(A, R, A.first);
+        if (kv == 0) quant_keys<DT, VEC>(A, R, b, h, 0, A.gh);
+        else quant_values<DT, VEC>(A, R, b, h, 0, A.gh * KG);
+        __syncthreads();
+        pass.store(A, R, A.first);
+        // further rows, each pass read whole before any of it is written: its destinations lie
+        // below the sources of every later pass
+        for (int r0 = A.first + COPY; r0 < A.keep; r0 += COPY) {
+            __syncthreads();
+            pass.load(A, R, r0);
+            __syncthreads();
+            pass.store(A, R, r0);
+        }
+    } else if (u < A.nhead + A.nbulk) {
+        const int t0 = A.gh * KG + (u - A.nhead) * BULK, t1 = min(t0 + BULK, A.ntok);
+        if (kv == 0) quant_keys<DT, VEC>(A, R, b, h, t0 / KG, t1 / KG);
+        else quant_values<DT, VEC>(A, R, b, h, t0, t1);
+    } else {
+        const int r0 = A.first + (u - A.nhead - A.nbulk) * COPY;
+        pass.load(A, R, r0);
+        pass.store(A, R, r0);
+    }
+}
+
+// Fills in the workgroups of an append of ntok quantized tokens and residual rows
+// [first, keep), and launches it (D divides 256 and is a multiple of 32).
+int launch_append(AppendArgs &A, int dtype, hipStream_t st, const char *who) {
+    const int na = A.src[A.kv0].na;
+    const bool in_place = A.ntok > 0 && na > 0;   // quantized groups read rows that the residual replaces
+    A.gh = in_place ? std::min((na + KG - 1) / KG, A.ntok / KG) : 0;
+    A.nhead = in_place ? 1 : 0;
+    A.nbulk = (A.ntok - A.gh * KG + BULK - 1) / BULK;
+    const int ncopy = in_place ? 0 : std::max(0, (A.keep - A.first + COPY - 1) / COPY);
+    const int64_t wgs = (int64_t)(A.nhead + A.nbulk + ncopy) * A.lanes * A.nkv;
+    if (wgs == 0) return MA_OK;
+    // 16-byte loads and stores: aligned bases and rows of whole 16-byte pieces
+    bool vec = true;
+    for (int kv = A.kv0; kv < A.kv0 + A.nkv; ++kv) {
+        const ma_tensor4 *ts[2] = {&A.src[kv].a, &A.src[kv].b};
+        for (const ma_tensor4 *t : ts) {
+            const int64_t m = dtype == MA_F32 ? 4 : 8;
+            if (t->ptr && (((uintptr_t)t->ptr & 15) || t->s[0] % m || t->s[1] % m || t->s[2] % m)) vec = false;
+        }
+    }
+    const dim3 grid((unsigned)wgs);
+#define MA_APPEND(DT_)                                                                                           \
+    do {                                                                                                         \
+        if (vec) hipLaunchKernelGGL((append_packed_kernel<DT_, true>), grid, dim3(AP_NT), 0, st, A);             \
+        else hipLaunchKernelGGL((append_packed_kernel<DT_, false>), grid, dim3(AP_NT), 0, st, A);                \
+    } while (0)
+    if (dtype == MA_BF16) MA_APPEND(MA_BF16);
+    else if (dtype == MA_F16) MA_APPEND(MA_F16);
+    else MA_APPEND(MA_F32);
+#undef MA_APPEND
+    return ma_check_launch(who);
+}
+
+// ---- quantizers of head dims that do not divide 256
+// DT: the dtype, a compile-time constant so that a thread's loads are straight-line code
+// (all of them in flight at once) instead of one branch per element
 // keys: grid (T/KG, B*H), D threads; thread = one channel of one token group.
 template <int DT>
-__global__ void quantize_keys_kernel(TwoSrc src, int H, int D, uint8_t *kq, int64_t q0, int64_t q1, int64_t q2,
+__global__ void quantize_keys_kernel(ma_tensor4 src, int H, int D, uint8_t *kq, int64_t q0, int64_t q1, int64_t q2,
                                      int64_t q3, _Float16 *ks, _Float16 *kz, int64_t s0, int64_t s1, int64_t s2) {
     const int bh = blockIdx.y, b = bh / H, h = bh % H;
     const int g = blockIdx.x;
@@ -222,15 +501,14 @@ __global__ void quantize_keys_kernel(TwoSrc src, int H, int D, uint8_t *kq, int6
     float lo = INFINITY, hi = -INFINITY;
 #pragma unroll
     for (int t = 0; t < KG; ++t) {
-        x[t] = two_load<DT>(src, b, h, g * KG + t, d);
+        x[t] = ma_load_f(src.ptr, b * src.s[0] + h * src.s[1] + (int64_t)(g * KG + t) * src.s[2] + d, DT);
         lo = fminf(lo, x[t]);
         hi = fmaxf(hi, x[t]);
     }
-    constexpr int dtype = DT;
-    QuantGroup qp = quant_params(lo, hi, dtype);
+    QuantGroup qp = quant_params(lo, hi, DT);
     uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
-    for (int t = 0; t < KG; ++t) w[t >> 3] |= quant_code(x[t], qp, dtype) << ((t & 7) * 4);
+    for (int t = 0; t < KG; ++t) w[t >> 3] |= quant_code(x[t], qp, DT) << ((t & 7) * 4);
     uint4 out = {w[0], w[1], w[2], w[3]};
     *(uint4 *)(kq + b * q0 + h * q1 + (int64_t)g * q2 + (int64_t)d * q3) = out;
     int64_t so = b * s0 + h * s1 + (int64_t)g * s2 + d;
@@ -240,13 +518,12 @@ __global__ void quantize_keys_kernel(TwoSrc src, int H, int D, uint8_t *kq, int6
 
 // values: one thread per (token, channel group); grid-stride over B*H*T*(D/VG) items.
 template <int DT>
-__global__ void __launch_bounds__(256) quantize_values_kernel(TwoSrc src, int BH, int H, int T, int D, uint8_t *vq,
-                                                              int64_t q0, int64_t q1, int64_t q2, int64_t q3,
-                                                              _Float16 *vs, _Float16 *vz, int64_t s0, int64_t s1,
-                                                              int64_t s2) {
+__global__ void __launch_bounds__(256) quantize_values_kernel(ma_tensor4 src, int BH, int H, int T, int D,
+                                                              uint8_t *vq, int64_t q0, int64_t q1, int64_t q2,
+                                                              int64_t q3, _Float16 *vs, _Float16 *vz, int64_t s0,
+                                                              int64_t s1, int64_t s2) {
     const int ncg = D / VG;
     const int64_t total = (int64_t)BH * T * ncg;
-    constexpr int dtype = DT;
     for (int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x; it < total; it += (int64_t)gridDim.x * 256) {
         int cg = (int)(it % ncg);
         int64_t rest = it / ncg;
@@ -256,14 +533,14 @@ __global__ void __launch_bounds__(256) quantize_values_kernel(TwoSrc src, int BH
         float lo = INFINITY, hi = -INFINITY;
 #pragma unroll
         for (int c = 0; c < VG; ++c) {
-            x[c] = two_load<DT>(src, b, h, j, cg * VG + c);
+            x[c] = ma_load_f(src.ptr, b * src.s[0] + h * src.s[1] + (int64_t)j * src.s[2] + cg * VG + c, DT);
             lo = fminf(lo, x[c]);
             hi = fmaxf(hi, x[c]);
         }
-        QuantGroup qp = quant_params(lo, hi, dtype);
+        QuantGroup qp = quant_params(lo, hi, DT);
         uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int c = 0; c < VG; ++c) w[c >> 3] |= quant_code(x[c], qp, dtype) << ((c & 7) * 4);
+        for (int c = 0; c < VG; ++c) w[c >> 3] |= quant_code(x[c], qp, DT) << ((c & 7) * 4);
         uint4 out = {w[0], w[1], w[2], w[3]};
         *(uint4 *)(vq + b * q0 + h * q1 + (int64_t)j * q2 + (int64_t)cg * q3) = out;
         int64_t so = b * s0 + h * s1 + (int64_t)j * s2 + cg;
@@ -272,66 +549,8 @@ __global__ void __launch_bounds__(256) quantize_values_kernel(TwoSrc src, int BH
     }
 }
 
-// The residual an append keeps: token rows [move, na + T) of [a | b] into a's rows
-// [0, keep), for K (blockIdx.y 0) and V (1).  Rows of a move down by `move` in place, so
-// one workgroup per lane copies them in chunks of CH rows, every chunk read whole before
-// any of it is written: a chunk's destination rows lie below the source rows of every
-// later chunk.  (move = 0 leaves a's rows where they are and appends b's.)
-constexpr int RK_NT = 256;
-template <int DT>
-__global__ void __launch_bounds__(RK_NT) residual_keep_kernel(TwoSrc k, TwoSrc v, int H, int D, int move, int keep) {
-    const TwoSrc &s = blockIdx.y ? v : k;
-    const int bh = blockIdx.x, b = bh / H, h = bh % H;
-    const int first = move == 0 ? s.na : 0;      // move = 0: a's rows stay, b's follow them
-    const int per = RK_NT / D;                   // rows per pass of the workgroup
-    const int r0 = threadIdx.x / D, d = threadIdx.x % D;
-    constexpr int RPT = 32;                      // rows per thread per chunk (64 rows at D = 128)
-    char *dst = (char *)s.a.ptr;
-    for (int c0 = first; c0 < keep; c0 += per * RPT) {
-        float x[RPT];
-#pragma unroll
-        for (int e = 0; e < RPT; ++e) {
-            const int r = c0 + e * per + r0;
-            x[e] = r < keep && r0 < per ? two_load<DT>(s, b, h, r + move, d) : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < RPT; ++e) {
-            const int r = c0 + e * per + r0;
-            if (r < keep && r0 < per)
-                ma_store_f(dst, b * s.a.s[0] + h * s.a.s[1] + (int64_t)r * s.a.s[2] + d, DT, x[e]);
-        }
-        __syncthreads();
-    }
-}
-
-template <int DT>
-void quant_keys_as(dim3 grid, int D, hipStream_t st, const TwoSrc &src, int H, void *kq, const int64_t *skq, void *ks,
-                   void *kz, const int64_t *sks) {
-    hipLaunchKernelGGL(quantize_keys_kernel<DT>, grid, dim3(D), 0, st, src, H, D, (uint8_t *)kq, skq[0], skq[1], skq[2],
-                       skq[3], (_Float16 *)ks, (_Float16 *)kz, sks[0], sks[1], sks[2]);
-}
-
-void launch_quant_keys(int dtype, dim3 grid, int D, hipStream_t st, const TwoSrc &src, int H, void *kq,
-                       const int64_t *skq, void *ks, void *kz, const int64_t *sks) {
-    if (dtype == MA_BF16) quant_keys_as<MA_BF16>(grid, D, st, src, H, kq, skq, ks, kz, sks);
-    else if (dtype == MA_F16) quant_keys_as<MA_F16>(grid, D, st, src, H, kq, skq, ks, kz, sks);
-    else quant_keys_as<MA_F32>(grid, D, st, src, H, kq, skq, ks, kz, sks);
-}
-
-template <int DT>
-void quant_values_as(int blocks, hipStream_t st, const TwoSrc &src, int BH, int H, int T, int D, void *vq,
-                     const int64_t *svq, void *vs, void *vz, const int64_t *svs) {
-    hipLaunchKernelGGL(quantize_values_kernel<DT>, dim3(blocks), dim3(256), 0, st, src, BH, H, T, D, (uint8_t *)vq,
-                       svq[0], svq[1], svq[2], svq[3], (_Float16 *)vs, (_Float16 *)vz, svs[0], svs[1], svs[2]);
-}
-
-void launch_quant_values(int dtype, int blocks, hipStream_t st, const TwoSrc &src, int BH, int H, int T, int D,
-                         void *vq, const int64_t *svq, void *vs, void *vz, const int64_t *svs) {
-    if (dtype == MA_BF16) quant_values_as<MA_BF16>(blocks, st, src, BH, H, T, D, vq, svq, vs, vz, svs);
-    else if (dtype == MA_F16) quant_values_as<MA_F16>(blocks, st, src, BH, H, T, D, vq, svq, vs, vz, svs);
-    else quant_values_as<MA_F32>(blocks, st, src, BH, H, T, D, vq, svq, vs, vz, svs);
-}
+// the head dims whose rows the append kernel's 256 threads share evenly
+bool append_dim(int D) { return D > 0 && D % VG == 0 && D <= AP_NT && AP_NT % D == 0; }
 
 }  // namespace
 
@@ -442,9 +661,29 @@ extern "C" int ma_quantize_keys(ma_tensor4 src, int B, int H, int T, int D, int 
         return MA_EINVAL;
     }
     if (T == 0) return MA_OK;
+    if (append_dim(D)) {
+        AppendArgs A{};
+        A.src[0] = TwoSrc{src, src, 0};
+        A.q[0] = (uint8_t *)kq;
+        A.s[0] = (_Float16 *)ks;
+        A.z[0] = (_Float16 *)kz;
+        std::copy(skq, skq + 4, A.sq[0]);
+        std::copy(sks, sks + 3, A.ss[0]);
+        A.H = H;
+        A.D = D;
+        A.lanes = B * H;
+        A.nkv = 1;
+        A.ntok = T;
+        return launch_append(A, src.dtype, (hipStream_t)stream, "ma_quantize_keys");
+    }
     dim3 grid(T / KG, B * H);
-    const TwoSrc two{src, src, 0};
-    launch_quant_keys(src.dtype, grid, D, (hipStream_t)stream, two, H, kq, skq, ks, kz, sks);
+#define MA_QK(DT_)                                                                                                    \
+    hipLaunchKernelGGL(quantize_keys_kernel<DT_>, grid, dim3(D), 0, (hipStream_t)stream, src, H, D, (uint8_t *)kq,    \
+                       skq[0], skq[1], skq[2], skq[3], (_Float16 *)ks, (_Float16 *)kz, sks[0], sks[1], sks[2])
+    if (src.dtype == MA_BF16) MA_QK(MA_BF16);
+    else if (src.dtype == MA_F16) MA_QK(MA_F16);
+    else MA_QK(MA_F32);
+#undef MA_QK
     return ma_check_launch("ma_quantize_keys");
 }
 
@@ -460,11 +699,33 @@ extern "C" int ma_quantize_values(ma_tensor4 src, int B, int H, int T, int D, in
         return MA_EINVAL;
     }
     if (T == 0) return MA_OK;
+    if (append_dim(D)) {
+        AppendArgs A{};
+        A.src[1] = TwoSrc{src, src, 0};
+        A.q[1] = (uint8_t *)vq;
+        A.s[1] = (_Float16 *)vs;
+        A.z[1] = (_Float16 *)vz;
+        std::copy(svq, svq + 4, A.sq[1]);
+        std::copy(svs, svs + 3, A.ss[1]);
+        A.H = H;
+        A.D = D;
+        A.lanes = B * H;
+        A.kv0 = 1;
+        A.nkv = 1;
+        A.ntok = T;
+        return launch_append(A, src.dtype, (hipStream_t)stream, "ma_quantize_values");
+    }
     int64_t items = (int64_t)B * H * T * (D / VG);
     int blocks = (int)((items + 255) / 256);
     if (blocks > 65535) blocks = 65535;
-    const TwoSrc two{src, src, 0};
-    launch_quant_values(src.dtype, blocks, (hipStream_t)stream, two, B * H, H, T, D, vq, svq, vs, vz, svs);
+#define MA_QV(DT_)                                                                                                    \
+    hipLaunchKernelGGL(quantize_values_kernel<DT_>, dim3(blocks), dim3(256), 0, (hipStream_t)stream, src, B * H, H,   \
+                       T, D, (uint8_t *)vq, svq[0], svq[1], svq[2], svq[3], (_Float16 *)vs, (_Float16 *)vz, svs[0],   \
+                       svs[1], svs[2])
+    if (src.dtype == MA_BF16) MA_QV(MA_BF16);
+    else if (src.dtype == MA_F16) MA_QV(MA_F16);
+    else MA_QV(MA_F32);
+#undef MA_QV
     return ma_check_launch("ma_quantize_values");
 }
 
@@ -474,7 +735,7 @@ extern "C" int ma_append_packed(ma_tensor4 k_res, ma_tensor4 v_res, int old_res,
                                 void *vz, const int64_t svs[3], void *stream) {
     const char *who = "ma_append_packed";
     if (B <= 0 || H <= 0 || T <= 0 || old_res < 0 || move < 0 || keep < 0 || move % KG || move + keep != old_res + T ||
-        D <= 0 || D % VG || D > RK_NT || RK_NT % D || !k_new.ptr || !v_new.ptr ||
+        !append_dim(D) || !k_new.ptr || !v_new.ptr ||
         ((old_res > 0 || keep > 0) && (!k_res.ptr || !v_res.ptr))) {
         ma_set_error("%s: bad geometry (move %% 32, move + keep = old_res + T, D | 256)", who);
         return MA_EINVAL;
@@ -484,35 +745,32 @@ extern "C" int ma_append_packed(ma_tensor4 k_res, ma_tensor4 v_res, int old_res,
         ma_set_error("%s: the residual and the new tokens must share one 16-bit or f32 dtype", who);
         return MA_EINVAL;
     }
-    const TwoSrc tk{k_res, k_new, old_res}, tv{v_res, v_new, old_res};
+    AppendArgs A{};
     if (move) {
         if (!kq || !ks || !kz || !skq || !sks || !vq || !vs || !vz || !svq || !svs || ((uintptr_t)kq & 15) ||
             ((uintptr_t)vq & 15) || ((skq[2] | skq[3] | svq[2] | svq[3]) & 15)) {
             ma_set_error("%s: packed planes missing or payload rows not 16-byte aligned", who);
             return MA_EINVAL;
         }
-        launch_quant_keys(k_new.dtype, dim3(move / KG, B * H), D, (hipStream_t)stream, tk, H, kq, skq, ks, kz, sks);
-        int rc = ma_check_launch(who);
-        if (rc) return rc;
-        const int64_t items = (int64_t)B * H * move * (D / VG);
-        int blocks = (int)((items + 255) / 256);
-        if (blocks > 65535) blocks = 65535;
-        launch_quant_values(k_new.dtype, blocks, (hipStream_t)stream, tv, B * H, H, move, D, vq, svq, vs, vz, svs);
-        rc = ma_check_launch(who);
-        if (rc) return rc;
+        A.q[0] = (uint8_t *)kq;
+        A.q[1] = (uint8_t *)vq;
+        A.s[0] = (_Float16 *)ks;
+        A.z[0] = (_Float16 *)kz;
+        A.s[1] = (_Float16 *)vs;
+        A.z[1] = (_Float16 *)vz;
+        std::copy(skq, skq + 4, A.sq[0]);
+        std::copy(svq, svq + 4, A.sq[1]);
+        std::copy(sks, sks + 3, A.ss[0]);
+        std::copy(svs, svs + 3, A.ss[1]);
     }
-    if (keep > (move ? 0 : old_res)) {
-        const dim3 grid(B * H, 2);
-        if (k_new.dtype == MA_BF16)
-            hipLaunchKernelGGL(residual_keep_kernel<MA_BF16>, grid, dim3(RK_NT), 0, (hipStream_t)stream, tk, tv, H, D,
-                               move, keep);
-        else if (k_new.dtype == MA_F16)
-            hipLaunchKernelGGL(residual_keep_kernel<MA_F16>, grid, dim3(RK_NT), 0, (hipStream_t)stream, tk, tv, H, D,
-                               move, keep);
-        else
-            hipLaunchKernelGGL(residual_keep_kernel<MA_F32>, grid, dim3(RK_NT), 0, (hipStream_t)stream, tk, tv, H, D,
-                               move, keep);
-        return ma_check_launch(who);
-    }
-    return MA_OK;
+    A.src[0] = TwoSrc{k_res, k_new, old_res};
+    A.src[1] = TwoSrc{v_res, v_new, old_res};
+    A.H = H;
+    A.D = D;
+    A.lanes = B * H;
+    A.nkv = 2;
+    A.ntok = move;
+    A.keep = keep;
+    A.first = move ? 0 : old_res;   // nothing quantized: the residual's rows stay, the new ones follow
+    return launch_append(A, k_new.dtype, (hipStream_t)stream, who);
 }

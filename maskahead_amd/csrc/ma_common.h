@@ -125,6 +125,12 @@ enum { MA_DPP_SHL1 = 0x101, MA_DPP_SHL2 = 0x102, MA_DPP_SHL4 = 0x104, MA_DPP_SHL
        MA_DPP_SHR1 = 0x111, MA_DPP_SHR2 = 0x112, MA_DPP_SHR4 = 0x114, MA_DPP_SHR8 = 0x118,
        MA_DPP_BCAST15 = 0x142, MA_DPP_BCAST31 = 0x143 };
 
+// the value of another lane of the quad (CTRL: quad_perm; 0xB1 = lane ^ 1, 0x4E = lane ^ 2)
+template <int CTRL>
+__device__ __forceinline__ float ma_quad(float x) {
+    return __uint_as_float(ma_dpp<CTRL>(__float_as_uint(x)));
+}
+
 // inclusive prefix sum over the 64 lanes of the wave (lane i gets lanes 0..i); u32 wraps
 __device__ __forceinline__ uint32_t ma_wave_prefix_u32(uint32_t x) {
     x += ma_dpp<MA_DPP_SHR1>(x);
