@@ -13,35 +13,13 @@ import torch
 
 from .. import _native as N
 from .select import _state
-from .splitk import Prefix, splitk_attention
+from .splitk import Prefix
 
 
 def _unpacked(prefix: Prefix, r: int, query: torch.Tensor) -> bool:
     """Whether the reference reads this packed prefix through a copy unpacked to the
     query dtype (splitk.py:513-516), as splitk_attention does."""
     return bool(prefix.nq) and (r > 256 or prefix.n > 256) and query.dtype != torch.float32
-
-
-def _vround(prefix: Prefix, r: int, query: torch.Tensor) -> int:
-    """The dtype of that copy, as splitk_attention records it in its statistics (bf16
-    queries; an f16 copy is made and read instead, see _staged)."""
-    return N.dtype_code(query.dtype) if _unpacked(prefix, r, query) else 0
-
-
-def _staged(query, prefix, current_key, current_value, rows, k, value, scale, out_key, out_value):
-    """Step 0 as its stages, for f16 queries over an unpacked packed prefix: splitk_attention
-    makes the f16 copy the reference reads (K and V rounded f32 -> f16, then f16 -> bf16 at
-    every dot) and the scores, the read set and the gather read that copy."""
-    from .ops import gather_packed_kv
-    from .select import prefix_scores_topk
-
-    out, stats = splitk_attention(query, prefix, current_key, current_value, scaling=scale, want_prefix=True)
-    mass, score, idx = prefix_scores_topk(query, prefix, stats, rows, k, value=value,
-                                          rank="score" if value else "mass", scaling=scale)
-    if out_key is not None or out_value is not None:
-        gather_packed_kv(stats[3], idx, dtype=(out_key if out_key is not None else out_value).dtype,
-                         out_key=out_key, out_value=out_value)
-    return out, stats, mass, score, idx
 
 
 class Step0Buffers:
@@ -74,8 +52,9 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
     call.  rows: the selection rows (a host list -- 0 .. T2-1 in order needs no table --
     or an int32 device tensor).  out_key / out_value (optional): [B, Hkv, k, D] views the
     selected entries are gathered into (the layer's compact buffer).  workspace: where the
-    scratch workspace lives (default bufs); layers run one after another on a stream can
-    share one."""
+    scratch workspace lives (default bufs), the f16 copy of a packed prefix among it
+    (prefix_used names that copy: valid until the owner's next call); layers run one after
+    another on a stream can share one."""
     stream = N.stream_of(query)
     rows_key = rows if isinstance(rows, torch.Tensor) else tuple(rows)
     views = tuple(None if x is None else (x.data_ptr(), x.shape, x.stride(), x.dtype) for x in (out_key, out_value))
@@ -86,12 +65,14 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
     # mask are the ones it was built from)
     if (plan is not None and plan[0] is prefix and plan[1] is workspace and plan[2] == key
             and (plan[3] is rows_key if isinstance(rows_key, torch.Tensor) else plan[3] == rows_key)
-            and plan[4][5] is prefix.native()):
-        args, result = plan[4], plan[5]
+            and plan[6] is prefix.native()):
+        args, result, copy = plan[4], plan[5], plan[7]
         # the same shapes, strides and dtypes (the key): only the operands' addresses change
         args[0].ptr = query.data_ptr()
         if current_key.shape[2]:
             args[7].ptr, args[8].ptr = current_key.data_ptr(), current_value.data_ptr()
+        if copy is not None:
+            N.check(N.load().ma_dequant_prefix(*copy), "ma_dequant_prefix")
         N.check(N.load().ma_step0(*args), "ma_step0")
         return result
     if query.ndim != 4 or current_key.ndim != 4:
@@ -120,13 +101,22 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
         t2 = len(host)
     if t2 == 0:
         raise ValueError("q_rows cannot be empty")
-    if query.dtype == torch.float16 and _unpacked(prefix, r, query):
-        return _staged(query, prefix, current_key, current_value, rows, k, value,
-                       float(scaling) if scaling is not None else d ** -0.5, out_key, out_value)
     dev = query.device
-    nat = prefix.native()
-    vround = _vround(prefix, r, query)
-    used = prefix.with_vround(vround) if vround else prefix
+    stored = nat = prefix.native()
+    used, vround, copy = prefix, 0, None
+    if _unpacked(prefix, r, query):
+        if query.dtype == torch.float16:
+            # the f16 copy the reference reads (K and V rounded f32 -> f16, then f16 -> bf16 at
+            # every dot), made in the workspace owner's storage: as splitk_attention's, without
+            # an allocation and a Python call per stage (93 -> 70 us a layer at 8 192 tokens)
+            own = workspace or bufs
+            k16, v16 = (own.take(x, b * hkv * n * d, torch.float16, dev, (b, hkv, n, d)) for x in ("k16", "v16"))
+            used = Prefix.dense(k16, v16, mask=prefix.mask)
+            copy = (stored, b, hkv, d, N.t4(k16), N.t4(v16), stream)
+            nat = used.native()
+        else:
+            vround = N.dtype_code(query.dtype)
+            used = prefix.with_vround(vround)
     out = bufs.take("out", query.numel(), query.dtype, dev, tuple(query.shape))
     mp = bufs.take("mp", b * hkv * r, torch.float32, dev, (b, hkv, r))
     lp = bufs.take("lp", b * hkv * r, torch.float32, dev, (b, hkv, r))
@@ -134,7 +124,7 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
     mass = bufs.take("mass", b * hkv * n, torch.float32, dev, (b, hkv, n))
     score = bufs.take("score", b * hkv * n, torch.float32, dev, (b, hkv, n)) if value else None
     idx = bufs.take("idx", b * hkv * k, torch.int64, dev, (b, hkv, k))
-    ws_bytes = N.size_query("ma_step0_workspace_bytes", b, hkv, hq, t, d, prefix.nq, prefix.nf)
+    ws_bytes = N.size_query("ma_step0_workspace_bytes", b, hkv, hq, t, d, used.nq, used.nf)
     if ws_bytes <= 0:
         raise N.KernelUnavailableError(f"ma_step0: no workspace size for n={n}")
     ws = (workspace or bufs).take("ws", ws_bytes, torch.uint8, dev, (ws_bytes,))
@@ -146,10 +136,12 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
             N.ptr(q_rows), t2, 1 if value else 0, 2 if value else 1, vround, mass.data_ptr(), N.ptr(score), k,
             idx.data_ptr(), N.t4(out_key), N.t4(out_value), st.data_ptr(), st.numel(), ws.data_ptr(), ws_bytes,
             stream]
+    if copy is not None:
+        N.check(N.load().ma_dequant_prefix(*copy), "ma_dequant_prefix")
     N.check(N.load().ma_step0(*args), "ma_step0")
     result = (out, (mp, lp, op, used), mass, score, idx)
     # the plan keeps every tensor its pointers name alive: q_rows (a cached device table, or
-    # None), the select state and the workspace (which another layer sharing the owner may
-    # have replaced by a larger one since)
-    bufs._plan = (prefix, workspace, key, rows_key, args, result, q_rows, st, ws)
+    # None), the select state, the workspace and the f16 copy (which another layer sharing
+    # the owner may have replaced by larger ones since)
+    bufs._plan = (prefix, workspace, key, rows_key, args, result, stored, copy, q_rows, st, ws)
     return result

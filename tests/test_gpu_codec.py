@@ -109,3 +109,30 @@ def test_quantizers_match_reference_golden(gpu, tag):
     assert np.array_equal(u16(ks), z[f"q_{tag}_ks"]) and np.array_equal(u16(kz), z[f"q_{tag}_kz"])
     assert np.array_equal(vq.cpu().numpy(), z[f"q_{tag}_vq"])
     assert np.array_equal(u16(vs), z[f"q_{tag}_vs"]) and np.array_equal(u16(vz), z[f"q_{tag}_vz"])
+
+
+@pytest.mark.parametrize("d,n,tail,pad", [(128, 288, 45, 0), (64, 96, 0, 0), (128, 0, 130, 0), (128, 160, 33, 5),
+                                          (64, 416, 1, 5)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_dequant_prefix_edges(gpu, d, n, tail, pad, dtype):
+    """Tiles of 128 tokens that hold packed, 16-bit or both parts, and outputs whose rows
+    allow no 16-byte stores (pad), in every output dtype."""
+    import ctypes
+
+    from maskahead_amd import _native as N
+
+    _, k, v, _, _ = layer_inputs(hq=4, hkv=2, d=d, n=n + tail, t=4, seed=23, dtype=torch.bfloat16)
+    want = [torch.empty((1, 2, 0, d))] * 2
+    if n:
+        store, nq = packed_cpu(k[:, :, :n], v[:, :, :n], pad_groups=1, pad_tokens=3)
+        want = list(dequant_cpu(store, nq))
+        p = gpu_prefix(store, nq, gpu, kf=k[:, :, n:] if tail else None, vf=v[:, :, n:] if tail else None)
+    else:
+        p = Prefix.dense(k.to(gpu), v.to(gpu))
+    want = [torch.cat([w, x[:, :, n:].float()], 2).to(dtype) for w, x in zip(want, (k, v))]
+    outs = [torch.full((1, 2, n + tail, d + pad), 7.0, dtype=dtype, device=gpu) for _ in range(2)]
+    ko, vo = (o[..., :d] for o in outs)
+    N.check(N.load().ma_dequant_prefix(ctypes.byref(p.native()), 1, 2, d, N.t4(ko), N.t4(vo), N.stream_of(ko)),
+            "ma_dequant_prefix")
+    assert torch.equal(ko.cpu(), want[0]) and torch.equal(vo.cpu(), want[1])
+    assert pad == 0 or all(torch.all(o[..., d:].cpu() == 7.0) for o in outs)

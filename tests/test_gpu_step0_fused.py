@@ -110,3 +110,34 @@ def test_step0_fused_errors(gpu):
         step0_select(bufs, q, p, kc, vc, list(range(32)), 2000, value=True)
     with pytest.raises(ValueError):
         step0_select(bufs, q, p, kc, vc, [40], 10, value=True)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_f16_step0_equals_its_stages(gpu, masked):
+    """f16 queries over a packed prefix with a residual, read through the f16 copy kept in
+    the workspace: a first call, a repeated one with other operands (the kept arguments) and
+    one of a second layer sharing the workspace equal the separate calls bit for bit."""
+    n, t, k = 320 + 21, 16, 64
+    ws = Step0Buffers()
+    layers = []
+    for seed in (5, 6):
+        q, kk, v, kc, vc = layer_inputs(hq=8, hkv=2, d=64, n=n, t=t, seed=seed, dtype=torch.bfloat16)
+        store, nq = packed_cpu(kk[:, :, :320], v[:, :, :320])
+        mask = None
+        if masked:
+            g = torch.Generator().manual_seed(seed)
+            mask = (torch.rand((1, 2, n), generator=g) > 0.2).to(torch.uint8)
+        p = gpu_prefix(store, nq, gpu, kf=kk[:, :, 320:].half(), vf=v[:, :, 320:].half(), mask=mask)
+        ops = [tuple((x * s).half().to(gpu) for x in (q, kc, vc)) for s in (1.0, 0.5)]
+        layers.append((Step0Buffers(), p, ops, [torch.empty((1, 2, k, 64), dtype=torch.float16, device=gpu) for _ in "kv"]))
+    for call in range(2):
+        for bufs, p, ops, (ck, cv) in layers:
+            q, kc, vc = ops[call]
+            out, stats, mass, score, idx = step0_select(bufs, q, p, kc, vc, list(range(t)), k, value=True, out_key=ck,
+                                                        out_value=cv, workspace=ws)
+            o2, st2 = splitk_attention(q, p, kc, vc, want_prefix=True)
+            m2, s2, i2 = prefix_scores_topk(q, p, st2, list(range(t)), k, value=True)
+            k2, v2 = gather_packed_kv(st2[3], i2, dtype=torch.float16)
+            for x, y in ((out, o2), (stats[0], st2[0]), (stats[1], st2[1]), (stats[2], st2[2]), (mass, m2), (score, s2),
+                         (idx, i2), (ck, k2), (cv, v2)):
+                assert torch.equal(x, y)
