@@ -34,8 +34,9 @@ struct FwdArgs {
     ma_tensor4 kc, vc;
     int H, G, T, R, Tc, nsplit, split_n, causal, q_pos0, c_pos0, row_tiles, row_groups, BH;
     // this launch: splits [0, nsp) of its token range [tok_beg, tok_end) of every lane,
-    // written to slots slot0 + split; with_cur: the current-block workgroups follow
-    int nsp, slot0, tok_beg, tok_end, with_cur;
+    // written to slots slot0 + split; with_tail: then the workgroups of a packed prefix's
+    // tail, tokens [tok_end, tail_end) to slot slot0 + nsp; with_cur: then the current block's
+    int nsp, slot0, tok_beg, tok_end, with_tail, tail_end, with_cur;
     float sl2;  // scale * log2(e)
     float scale;
     // partials of every (lane, slot, row), slot = split or nsplit (current block):
@@ -125,23 +126,35 @@ __device__ __forceinline__ void s_qk(const uint16_t *K, const bf16x8_t *qf, int 
     }
 }
 
-// Workgroup index -> (segment, lane bh, row group, split).  Prefix splits first, the
-// current-block workgroups last (they are short, so they fill in behind the splits).
+// Workgroup index -> (segment, lane bh, row group, split).  Prefix splits first, then the
+// packed prefix's tail and the current block (short, so they fill in behind the splits).
+enum { SEG_SPLIT = 0, SEG_TAIL = 1, SEG_CUR = 2 };
 struct Work {
+    int seg;
     bool cur;
     int bh, rg, sp;
 };
 
+template <int SRC>
 __device__ __forceinline__ Work decode_work(const FwdArgs &a) {
     Work w;
     int idx = blockIdx.x;
     const int npre = a.nsp * a.BH * a.row_groups;
-    w.cur = idx >= npre;
-    if (w.cur) idx -= npre;
+    w.seg = SEG_SPLIT;
+    if (idx >= npre) {
+        idx -= npre;
+        w.seg = SEG_CUR;
+        if (SRC == 0 && a.with_tail) {
+            const int ntail = a.BH * a.row_groups;
+            if (idx < ntail) w.seg = SEG_TAIL;
+            else idx -= ntail;
+        }
+    }
+    w.cur = w.seg == SEG_CUR;
     w.rg = idx % a.row_groups;
     idx /= a.row_groups;
     w.bh = idx % a.BH;
-    w.sp = w.cur ? 0 : idx / a.BH;
+    w.sp = w.seg == SEG_SPLIT ? idx / a.BH : 0;
     return w;
 }
 
@@ -310,27 +323,39 @@ __device__ __forceinline__ void pv_regs(const uint16_t *Vt, const bf16x8_t *pb, 
             acc[dt] = ma_mfma32(*(const bf16x8_t *)&vrow[dt * 32 * VS + c * 16], pb[c], acc[dt]);
 }
 
-// The current block of one (lane, row group) for the packed kernel: its tiles staged
-// synchronously by every thread from the 16-bit current K/V, then S^T, softmax
-// (block-causal mask) and PV; the partial goes to slot nsplit.
+// A short segment of one (lane, row group) of the packed kernel, its tiles staged
+// synchronously by every thread, then S^T, softmax and PV:
+//   the current block (block-causal mask), partial to slot nsplit;
+//   the packed prefix's tail: what its whole 64-token tiles leave, an odd key group of 32
+//   tokens and the 16-bit residual, partial to the slot behind the splits.
 template <int D>
-__device__ __forceinline__ void cur_segment(const FwdArgs &a, const Work &wk, FwdSmem<D> &S) {
+__device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, const Lane &L, FwdSmem<D> &S) {
     constexpr int NKS = D / 16;
     constexpr int NDT = D / 32;
     const int bh = wk.bh, b = bh / a.H, h = bh % a.H;
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, c32 = lane & 31, hf = lane >> 5;
-    const Dense kc = dense_lane(a.kc.ptr, a.kc.s, a.kc.dtype, b, h);
-    const Dense vc = dense_lane(a.vc.ptr, a.vc.s, a.vc.dtype, b, h);
-    const int Tc = a.Tc;
-    const int nt = (Tc + TILE - 1) / TILE;
+    const bool cur = wk.cur;
+    Dense kc, vc;
+    if (cur) {
+        kc = dense_lane(a.kc.ptr, a.kc.s, a.kc.dtype, b, h);
+        vc = dense_lane(a.vc.ptr, a.vc.s, a.vc.dtype, b, h);
+    } else {
+        kc = Dense{L.kf, L.kf_n, L.fdtype, L.esz};
+        vc = Dense{L.vf, L.vf_n, L.fdtype, L.esz};
+    }
+    const int beg = cur ? 0 : a.tok_end;                   // first token of the segment
+    const int ntok = cur ? a.Tc : a.tail_end - beg;
+    const int np = cur ? 0 : L.nq - beg;                   // its packed tokens: 0 or one group
+    const uint8_t *mask = cur ? nullptr : L.mask;
+    const int nt = (ntok + TILE - 1) / TILE;
     const int nS = min(MAXS, a.row_tiles - wk.rg * MAXS);
     const bool is_s = wave < nS;
     const int rtile = wk.rg * MAXS + wave;
     const int row = rtile * 32 + c32;
     const bool row_ok = row < a.R;
     const int qpos = a.q_pos0 + (row_ok ? row % a.T : 0);
-    const bool causal = a.causal > 0;
+    const bool causal = cur && a.causal > 0;
     bf16x8_t qf[NKS];
     if (is_s) {
         const int g = row_ok ? row / a.T : 0, t = row_ok ? row % a.T : 0;
@@ -346,21 +371,42 @@ __device__ __forceinline__ void cur_segment(const FwdArgs &a, const Work &wk, Fw
     for (int dt = 0; dt < NDT; ++dt) acc[dt] = f32x16_t{};
     for (int i = 0; i < nt; ++i) {
         const int n0 = i * TILE;
-        const int valid = Tc - n0;
+        const int valid = ntok - n0;
+        const int pk = i == 0 ? np : 0;                    // packed tokens of this tile
         uint32_t w[8];
-        const char *kb = kc.base + (int64_t)n0 * kc.sn * kc.esz;
+        if (pk) {
+            for (int u = tid; u < D; u += NTH) {           // the items of key group 0 of the tile
+                load_k_packed<D>(w, L, u, beg, L.nq);
+                store_k_packed<D>(S.u.t.kt[0].k, w, u);
+            }
+            for (int u = tid; u < 2 * D; u += NTH) {
+                if ((u & 31) >= KGRP / 2) continue;        // token pairs of the group
+                uint32_t fl;
+                load_v_packed<D>(w, fl, L, u, beg, L.nq);
+                store_v_packed<D>(S.u.t.vt[0].vt, w, u);
+            }
+        }
+        // 16-bit tokens [pk, valid) of the tile; tokens from `valid` on are staged as zeros
+        const int64_t r0 = n0 - np;                        // row of the tile's first token
+        const char *kb = kc.base + r0 * kc.sn * kc.esz;
         for (int u = tid; u < TILE * D / 8; u += NTH) {
-            const bool ok = load_k_dense<D>(w, kb, kc.sn, kc.dtype, kc.esz, u, valid);
+            const int t = u / (D / 8);
+            if (t < pk) continue;
+            const bool ok = t < valid;
+            if (ok) load_k_dense<D>(w, kb, kc.sn, kc.dtype, kc.esz, u, valid);
             store_k_dense<D>(S.u.t.kt[0].k, w, u, kc.dtype, ok);
         }
-        const char *vb = vc.base + (int64_t)n0 * vc.sn * vc.esz;
+        const char *vb = vc.base + r0 * vc.sn * vc.esz;
         for (int u = tid; u < TILE / 2 * D / 8; u += NTH) {
-            const int tp = u % (TILE / 2);
-            load_v_dense<D>(w, vb, vc.sn, vc.dtype, vc.esz, u, valid);
-            store_v_dense<D>(S.u.t.vt[0].vt, w, u, vc.dtype, 2 * tp < valid, 2 * tp + 1 < valid);
+            const int t = 2 * (u % (TILE / 2));
+            if (t < pk) continue;
+            const bool l0 = t < valid && (!mask || mask[beg + n0 + t]);
+            const bool l1 = t + 1 < valid && (!mask || mask[beg + n0 + t + 1]);
+            if (t < valid) load_v_dense<D>(w, vb, vc.sn, vc.dtype, vc.esz, u, valid);
+            store_v_dense<D>(S.u.t.vt[0].vt, w, u, vc.dtype, l0, l1);
         }
         if (wave == 0) {
-            const uint64_t m = __ballot(lane < valid);
+            const uint64_t m = __ballot(lane < valid && (!mask || mask[beg + n0 + min(lane, valid - 1)]));
             if (lane == 0) S.kmask[0] = m;
         }
         __syncthreads();  // tile staged
@@ -378,30 +424,32 @@ __device__ __forceinline__ void cur_segment(const FwdArgs &a, const Work &wk, Fw
         }
         __syncthreads();  // buffers free
     }
-    if (is_s) write_partial<D>(a, acc, m_ref, m_true, l, bh, a.nsplit, rtile, c32, hf, lane, &S.u.o[wave][0]);
+    if (is_s)
+        write_partial<D>(a, acc, m_ref, m_true, l, bh, cur ? a.nsplit : a.slot0 + a.nsp, rtile, c32, hf, lane,
+                         &S.u.o[wave][0]);
 }
 
-// FULL (packed only): no slot mask and every split a run of whole 64-token tiles (the host
-// checks nq % 64 == 0), so only the whole-tile staging path is built
-template <int D, int SRC, bool FULL>
+// MASK: the prefix has a slot mask (packed sources: their splits are whole 64-token tiles
+// either way, what is left goes to short_segment, so no tile needs bounds)
+template <int D, int SRC, bool MASK>
 __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
     __shared__ FwdSmem<D> S;
     using Shape = StageShape<KLANES, D, SRC == 0 ? ST_PACKED : ST_DENSE>;
     constexpr int NKS = D / 16;
     constexpr int NDT = D / 32;
 
-    const Work wk = decode_work(a);
-    if constexpr (SRC == 0) {
-        if (wk.cur) {
-            cur_segment<D>(a, wk, S);
-            return;
-        }
-    }
+    const Work wk = decode_work<SRC>(a);
     const int bh = wk.bh, b = bh / a.H, h = bh % a.H;
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, c32 = lane & 31, hf = lane >> 5;
 
     const Lane L = make_lane(a.pre, b, h, bh);
+    if constexpr (SRC == 0) {
+        if (wk.seg != SEG_SPLIT) {
+            short_segment<D>(a, wk, L, S);
+            return;
+        }
+    }
     int n_beg, n_end;
     if (wk.cur) {
         n_beg = 0;
@@ -455,7 +503,9 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
         if (is_k && kl < Shape::NK) item_off = k_item_offsets<D>(L, kl);
         else if (!is_k && vl < Shape::NV) item_off = v_item_offsets<D>(L, vl);
     }
-    const bool fast_tiles = SRC == 0 && (FULL || !L.mask);
+    // raw mask bytes of a packed tile in flight (this K lane's token; this V lane's pair),
+    // looked at only when the tile is staged
+    uint32_t mb0 = 1u, mb1 = 1u;
     // all-bf16 dense source without a slot mask: the byte offset of this thread's first
     // item from a whole tile's first token, computed once (a whole tile then costs one base
     // address per operand and no bounds checks).  Item r of a K lane is KLANES / (D / 8) * r
@@ -474,22 +524,15 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
     auto load_k = [&](int i) {
         const int n0 = tile_n0(i);
         if constexpr (SRC == 0) {
-            if (FULL || (fast_tiles && n0 + TILE <= n_end)) {
-                pr.flags = kl < TILE ? 256u : 0u;
-                if (kl < Shape::NK) {
-                    const int64_t g0 = n0 / KGRP;
-                    load_k_packed_fast(pr.w, L.kq + g0 * L.kq_g, L.ks + g0 * L.ks_g, L.kz + g0 * L.ks_g, L.kq_d,
-                                       item_off);
-                }
-                return;
+            if (kl < Shape::NK) {
+                const int64_t g0 = n0 / KGRP;
+                load_k_packed_fast(pr.w, L.kq + g0 * L.kq_g, L.ks + g0 * L.ks_g, L.kz + g0 * L.ks_g, L.kq_d, item_off);
             }
-        }
-        pr.flags = (kl < TILE && live(n0 + kl)) ? 256u : 0u;
-        if constexpr (SRC == 0) {
-            if constexpr (!FULL) {
-                if (kl < Shape::NK) load_k_packed<D>(pr.w, L, kl, n0, n_end);
+            if constexpr (MASK) {
+                if (kl < TILE) mb0 = L.mask[n0 + kl];
             }
         } else {
+            pr.flags = (kl < TILE && live(n0 + kl)) ? 256u : 0u;
             const char *base = ds.k + (int64_t)(n0 - ds.tok0) * ds.sk * ds.esz;
             if constexpr (SRC == 2) {
                 if (dense_fast && n0 + TILE <= n_end) {
@@ -527,23 +570,21 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
             }
         }
         if (kl < TILE) {
-            const uint64_t m = __ballot((pr.flags & 256u) != 0);
+            const uint64_t m = __ballot(SRC == 0 ? mb0 != 0 : (pr.flags & 256u) != 0);
             if (kl == 0) km = m;
         }
     };
     auto load_v = [&](int i) {
         const int n0 = tile_n0(i);
         if constexpr (SRC == 0) {
-            if (FULL || (fast_tiles && n0 + TILE <= n_end)) {
-                if (vl < Shape::NV) {
-                    load_v_packed_fast(pr.w, L.vq + (int64_t)n0 * L.vq_n, L.vs + (int64_t)n0 * L.vs_n,
-                                       L.vz + (int64_t)n0 * L.vs_n, L.vq_n, L.vs_n, item_off);
-                    pr.flags = 3u;
+            if (vl < Shape::NV) {
+                load_v_packed_fast(pr.w, L.vq + (int64_t)n0 * L.vq_n, L.vs + (int64_t)n0 * L.vs_n,
+                                   L.vz + (int64_t)n0 * L.vs_n, L.vq_n, L.vs_n, item_off);
+                if constexpr (MASK) {
+                    const uint8_t *m = L.mask + n0 + 2 * (vl & 31);
+                    mb0 = m[0];
+                    mb1 = m[1];
                 }
-                return;
-            }
-            if constexpr (!FULL) {
-                if (vl < Shape::NV) load_v_packed<D>(pr.w, pr.flags, L, vl, n0, n_end);
             }
         } else {
             const char *base = ds.v + (int64_t)(n0 - ds.tok0) * ds.sv * ds.esz;
@@ -584,6 +625,12 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
     };
     auto store_v = [&](uint16_t *Vt) {
         if constexpr (SRC == 0) {
+            if constexpr (MASK) {
+                // dead tokens stage zeros (codes, scale and zero), never stale NaN
+#pragma unroll
+                for (int e = 0; e < 8; ++e) pr.w[e] = ((e & 2) && e < 4) || (e >= 4 && (e & 1)) ? (mb1 ? pr.w[e] : 0u)
+                                                                                                 : (mb0 ? pr.w[e] : 0u);
+            }
             if (vl < Shape::NV) store_v_packed<D>(Vt, pr.w, vl);
         } else {
 #pragma unroll
@@ -650,7 +697,23 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
         const int cb = it % NBUF;
         const uint64_t mc = S.kmask[cb];
         if (is_s) {
-            if constexpr (!FULL) {
+            if constexpr (SRC == 0) {
+                if constexpr (MASK) {
+                    // the masked pass costs little over the plain one (6 997 tokens, 2 tiles a
+                    // workgroup: 18.8 us; with bounds, clamps and mask tests where the loads are
+                    // issued it needed a launch more for its tail, 28.3 us in all):
+                    // element i of half t2 is token t2 * 32 + (i >> 2) * 8 + hf * 4 + (i & 3): its
+                    // mask bit spread over the word selects the score or -inf (two operations)
+                    const uint32_t ok[2] = {(uint32_t)mc >> (hf * 4), (uint32_t)(mc >> 32) >> (hf * 4)};
+#pragma unroll
+                    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)ok[t2], (i >> 2) * 8 + (i & 3), 1);
+                            sc[t2][i] = __uint_as_float((keep & __float_as_uint(sc[t2][i])) | (~keep & 0xff800000u));
+                        }
+                }
+            } else {
                 const int n0 = tile_n0(it);
                 const int lim = causal ? (qpos / a.causal + 1) * a.causal - a.c_pos0 - n0 - hf * 4 : TILE;
                 if (causal || mc != ~0ull) {
@@ -805,17 +868,40 @@ __global__ void __launch_bounds__(128) splitk_combine_kernel(FwdArgs a, ma_tenso
     }
 }
 
+// The parts of a prefix: packed whole tiles [0, nq64) in splits, then -- packed prefixes --
+// the tail [nq64, tail_end), then the 16-bit part [tail_end, n) in splits of its own.  The
+// residual of a cache (fewer than 64 tokens, unless blocks are staged unquantized) joins the
+// tail: as a launch of its own, with the current block, it cost 9.5 us behind a packed pass
+// of 28 (8 workgroups, one tile each).  Longer 16-bit parts keep their own pipelined launch.
+constexpr int MAX_TAIL = 4 * TILE;
+struct Parts {
+    int nq64, tail_end;
+    int splits(int sn) const { return (nq64 + sn - 1) / sn; }
+    bool tail() const { return tail_end > nq64; }
+    int fsplits(int nq, int nf, int sn) const { return (nq + nf - tail_end + sn - 1) / sn; }
+};
+Parts parts_of(int nq, int nf) {
+    Parts p;
+    p.nq64 = nq / TILE * TILE;
+    p.tail_end = nq > 0 && nq + nf - p.nq64 <= MAX_TAIL ? nq + nf : nq;
+    return p;
+}
+
 // Tokens per split: about one workgroup per CU (a workgroup's 256 VGPRs per lane and
 // 108 KB of LDS fill a CU), with
-// one CU per (lane, row group) left for the current block's workgroups, so every
+// one CU per (lane, row group) left for the current block's workgroups, and one for a packed
+// prefix's tail, so every
 // workgroup of the launch runs in the first dispatch wave; at least one 64-token tile.
+// (Where many row groups leave few splits, a tail's CU would lengthen every split by a good
+// part; the tail then runs beside the splits of other CUs' second dispatch wave.)
 // Short prefixes (a sub-step's 2 048 selected entries) thus spread over many CUs: each
 // workgroup's cost is mostly fixed latency, so more, shorter splits finish sooner
 // (22.1 -> 17.9 us per sub-step at 4 KV heads x 2 048 entries, measured).
-int choose_split(int n, int BH, int row_groups, int split_tokens) {
+int choose_split(int nq, int nf, int BH, int row_groups, int split_tokens) {
     if (split_tokens > 0) return split_tokens;
-    const int units = BH * row_groups;
+    const int units = BH * row_groups, n = nq + nf;
     int per = ma_num_cus() / units - 1;
+    if (per > 8 && parts_of(nq, nf).tail()) --per;
     if (per < 1) per = 1;
     int sn = (n + per - 1) / per;
     sn = ((sn + TILE - 1) / TILE) * TILE;
@@ -829,9 +915,11 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 int ma_validate_prefix(const ma_prefix *p, int D, const char *who);
 
-// Slots of the partials: ceil(nq / sn) packed splits, ceil(nf / sn) 16-bit splits, then
-// the current block.
-static int slot_count(int nq, int nf, int sn) { return (nq + sn - 1) / sn + (nf + sn - 1) / sn; }
+// Slots of the partials: the packed splits, the tail, the 16-bit splits, then the current block.
+static int slot_count(int nq, int nf, int sn) {
+    const Parts p = parts_of(nq, nf);
+    return p.splits(sn) + (p.tail() ? 1 : 0) + p.fsplits(nq, nf, sn);
+}
 
 static int row_groups_of(int Hq, int H, int T) {
     const int row_tiles = ((Hq / H) * T + 31) / 32;
@@ -842,7 +930,7 @@ extern "C" int64_t ma_splitk_workspace_bytes(int B, int H, int Hq, int T, int D,
                                              int split_tokens) {
     if (B <= 0 || H <= 0 || Hq <= 0 || Hq % H || T <= 0 || D <= 0 || nq < 0 || nf < 0) return -1;
     const int R = (Hq / H) * T;
-    const int sn = choose_split(nq + nf, B * H, row_groups_of(Hq, H, T), split_tokens);
+    const int sn = choose_split(nq, nf, B * H, row_groups_of(Hq, H, T), split_tokens);
     const int nsplit = slot_count(nq, nf, sn);
     const int64_t rows = (int64_t)B * H * (nsplit + 1) * R;
     return rows * 4 * 3 + rows * D * 2 + 256;
@@ -888,8 +976,7 @@ int make_plan(Plan &pl, const char *who, ma_tensor4 q, int B, int Hq, int T, int
     const int R = G * T;
     const int row_tiles = (R + 31) / 32;
     const int row_groups = (row_tiles + MAXS - 1) / MAXS;
-    const int n = p->nq + p->nf;
-    const int sn = choose_split(n, B * H, row_groups, split_tokens);
+    const int sn = choose_split(p->nq, p->nf, B * H, row_groups, split_tokens);
     const int nsplit = slot_count(p->nq, p->nf, sn);
     const int64_t need = ma_splitk_workspace_bytes(B, H, Hq, T, D, p->nq, p->nf, sn);
     if (workspace_bytes < need) {
@@ -933,42 +1020,38 @@ int make_plan(Plan &pl, const char *who, ma_tensor4 q, int B, int Hq, int T, int
 
 template <int D>
 int launch_partial_d(const Plan &pl, hipStream_t st) {
-    // packed part [0, nq) and 16-bit part [nq, n) in a launch each; the current block is
-    // attended in the merge
+    // the packed splits with the tail in one launch, a 16-bit part beyond the tail in another;
+    // the current block's workgroups (last in the grid) ride with the last of them
     FwdArgs fa = pl.fa;
     const int nq = fa.pre.nq, nf = fa.pre.nf, sn = fa.split_n;
     const int units = pl.B * fa.H * pl.row_groups;
-    const int nsq = (nq + sn - 1) / sn, nsf = (nf + sn - 1) / sn;
-    // the current block's workgroups (last in the grid) ride with the packed launch when
-    // there is no 16-bit part, else with the 16-bit one
-    const bool cur_in_packed = nsq > 0 && nsf == 0;
-    if (nsq) {
+    const Parts pt = parts_of(nq, nf);
+    const int nsq = pt.splits(sn), nsf = pt.fsplits(nq, nf, sn);
+    fa.with_tail = pt.tail();
+    if (nq) {
         fa.nsp = nsq;
         fa.slot0 = 0;
         fa.tok_beg = 0;
-        fa.tok_end = nq;
-        fa.with_cur = cur_in_packed;
-        // whole tiles everywhere: no slot mask, a packed part of whole tiles (every split is)
-        const bool full = !fa.pre.mask && nq % TILE == 0;
-        if (full)
-            hipLaunchKernelGGL((splitk_fwd_kernel<D, 0, true>), dim3((nsq + fa.with_cur) * units), dim3(NTH), 0, st,
-                               fa);
-        else
-            hipLaunchKernelGGL((splitk_fwd_kernel<D, 0, false>), dim3((nsq + fa.with_cur) * units), dim3(NTH), 0,
-                               st, fa);
+        fa.tok_end = pt.nq64;
+        fa.tail_end = pt.tail_end;
+        fa.with_cur = nsf == 0;
+        const dim3 grid((nsq + fa.with_tail + fa.with_cur) * units);
+        if (fa.pre.mask) hipLaunchKernelGGL((splitk_fwd_kernel<D, 0, true>), grid, dim3(NTH), 0, st, fa);
+        else hipLaunchKernelGGL((splitk_fwd_kernel<D, 0, false>), grid, dim3(NTH), 0, st, fa);
     }
-    if (!cur_in_packed) {
+    if (!nq || nsf) {
+        fa.slot0 = nsq + fa.with_tail;
         fa.nsp = nsf;
-        fa.slot0 = nsq;
-        fa.tok_beg = nq;
+        fa.tok_beg = pt.tail_end;
         fa.tok_end = nq + nf;
+        fa.with_tail = 0;
         fa.with_cur = 1;
         const bool bf = (nf == 0 || fa.pre.fdtype == MA_BF16) &&
                         (fa.Tc == 0 || (fa.kc.dtype == MA_BF16 && fa.vc.dtype == MA_BF16));
         if (bf)
-            hipLaunchKernelGGL((splitk_fwd_kernel<D, 2, false>), dim3((nsf + 1) * units), dim3(NTH), 0, st, fa);
+            hipLaunchKernelGGL((splitk_fwd_kernel<D, 2, true>), dim3((nsf + 1) * units), dim3(NTH), 0, st, fa);
         else
-            hipLaunchKernelGGL((splitk_fwd_kernel<D, 1, false>), dim3((nsf + 1) * units), dim3(NTH), 0, st, fa);
+            hipLaunchKernelGGL((splitk_fwd_kernel<D, 1, true>), dim3((nsf + 1) * units), dim3(NTH), 0, st, fa);
     }
     return ma_check_launch("ma_splitk_partial");
 }
