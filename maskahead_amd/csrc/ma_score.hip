@@ -20,9 +20,9 @@
 //     per-thread offset fixed for the whole run and a wave-uniform tile base.
 //   * wave 15 (a staging wave) finishes tile i-1: sum over row tiles, live mask, mass and
 //     score.
-// "Tail" workgroups take one of the remaining tiles each (the tile that straddles a
-// packed prefix's 16-bit residual, 16-bit tail tiles, a partial last tile, f32 prefixes)
-// and stage it element-wise.  Both share a prologue that builds, once per workgroup, the
+// "Tail" workgroups take one of the remaining tiles each: the tile that straddles a
+// packed prefix's 16-bit residual and 16-bit tail tiles are staged by items, others (a
+// partial last tile of a 16-bit prefix, f32 prefixes) element-wise.  Both share a prologue that builds, once per workgroup, the
 // selection-row tables in LDS (row of every selection row, its query offset and c_r, one
 // load per row) and the value centre (mean of O_p over the selection rows, a fixed-order
 // LDS reduction shared with ma_value_centre).
@@ -55,6 +55,7 @@ struct ScoreArgs {
     int nfast;     // whole tiles of the source kind per lane: tiles [0, nfast)
     int per;       // tiles per fast workgroup
     int fast_wgs;  // fast workgroups per lane (blockIdx.x below it); then one tail tile each
+    int tail_vec;  // tail tiles of a packed prefix are staged by items (16-bit rows that allow it)
     float sl2;
     // the read-set top-k's level-0 histogram of this pass's ranks (ma_topk_select_hist_ready):
     // 0 none, 1 the mass, 2 the score of every slot (dead slots -inf), counted into
@@ -688,17 +689,58 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
     };
 
     if (!fast) {
-        // ---- tail workgroup: one tile, staged element-wise by every thread
+        // ---- tail workgroup: one tile, staged by items, or element-wise by every thread
         const Lane L = make_lane<LANE32 ? 1 : 0>(a.pre, b, h, bh);
         const int n0 = tile0 * TILE;
         uint16_t *Ks = sm.u.kt[0].k;
+        // A packed prefix's tail (an odd key group of 32 tokens, or none, then 16-bit rows) is
+        // staged by items: those of tokens 0 .. 31 are the ones below 2 D, so a 32-token half is
+        // either packed items or 16-bit ones; rows past the end repeat the last one (their
+        // results are not written).  (Element by element a tail was the longest workgroup of a
+        // short prefix: 544 tokens, 12.6 -> 11.4 us.)
+        if (SRC == SRC_PACKED && a.tail_vec) {
+            const int np = a.pre.nq - n0;   // packed tokens of the tile: 32, or none (<= 0)
+#pragma unroll
+            for (int j = 0; j < IPT; ++j) {
+                const int u = item(j), v = u % NIK;
+                if (u >= ni) continue;
+                uint32_t x[8];
+                float dd = 0.f;
+                const float *cen16 = &sm.cen[(v % TPI) * 16];
+                if (v / (2 * D) * KGRP < np) {
+                    const int64_t g = n0 / KGRP;
+                    if (u < NIK) {
+                        kp_load(x, L.kq + g * L.kq_g, L.ks + g * L.ks_g, L.kz + g * L.ks_g, L.kq_d, kp_offsets<D>(L, u));
+                        kp_store<D>(Ks, x, u);
+                    } else {
+                        vp_load(x, L.vq + (int64_t)n0 * L.vq_n, L.vs + (int64_t)n0 * L.vs_n,
+                                L.vz + (int64_t)n0 * L.vs_n, vp_offsets<D>(L, v));
+                        dd = a.vround == MA_BF16 ? vp_dist<MA_BF16>(x, cen16)
+                                                 : (a.vround == MA_F16 ? vp_dist<MA_F16>(x, cen16) : vp_dist<0>(x, cen16));
+                    }
+                } else if (a.pre.nf > 0) {   // (else no row to repeat: that half's results are not written)
+                    const int64_t r = min(n0 + v / TPI, end - 1) - a.pre.nq;
+                    if (u < NIK) {
+                        d32_load(x, L.kf + (r * L.kf_n + v % TPI * 16) * 2, 0u);
+                        kd_store<D>(Ks, x, u, a.pre.fdtype);
+                    } else {
+                        d32_load(x, L.vf + (r * L.vf_n + v % TPI * 16) * 2, 0u);
+                        dd = vd_dist(x, cen16, a.pre.fdtype);
+                    }
+                }
+                if (u >= NIK) {
+                    dd = token_sum<D>(dd);
+                    if (v % TPI == 0) sm.dist[0][v / TPI] = dd;
+                }
+            }
+        } else
 #pragma unroll 1
         for (int it = tid; it < TILE * D; it += NT) {
             const int t = it / D, d = it % D;
             const int j = n0 + t;
             Ks[t * KS + d] = ma_f32_to_bf16(j < end ? lane_key(L, j, d) : 0.f);
         }
-        if (value) {
+        if (value && !(SRC == SRC_PACKED && a.tail_vec)) {
             // V items (token, 16 channels), the D/16 lanes of a token adjacent
             for (int v0 = 0; v0 < NIK; v0 += NT) {
                 const int v = v0 + tid;
@@ -1161,8 +1203,13 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
     // f32 or unaligned 16-bit prefixes) to one tail workgroup each
     int nfast = packed ? p->nq / TILE : n / TILE;
     if (!dense_vec_ok) nfast = 0;
-    const int slots = wgs_per_cu * ma_num_cus();
-    int per = nfast > 0 ? (nfast * B * H + slots - 1) / slots : 1;
+    // whole tiles in runs of `per`, the tail tiles' workgroups beside them in the same dispatch
+    // wave: at 32 768 packed tokens + a residual, 64 runs of 8 tiles a lane and the tails
+    // behind them took 34.1 us, 57 runs of 9 take 25.9.  (A launch of many tails, an
+    // unaligned or f32 prefix, is theirs in any case.)
+    const int slots = wgs_per_cu * ma_num_cus(), ntail = (tiles - nfast) * B * H;
+    const int room = ntail * 4 <= slots ? slots - ntail : slots;
+    int per = nfast > 0 ? (nfast * B * H + room - 1) / room : 1;
     if (per < 1) per = 1;
     const int fast_wgs = nfast > 0 ? (nfast + per - 1) / per : 0;
     ScoreArgs sa{};
@@ -1237,6 +1284,7 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
         return ma_topk_level0_into_state(hist_rank == 2 ? score : mass, n, p->mask, n, B * H, n, topk_state, stream);
     }
     sa.nfast = nfast;
+    sa.tail_vec = packed && dense_vec_ok;
     sa.per = per;
     sa.fast_wgs = fast_wgs;
     dim3 grid(fast_wgs + (tiles - nfast), H, B);
