@@ -136,3 +136,22 @@ def test_dequant_prefix_edges(gpu, d, n, tail, pad, dtype):
             "ma_dequant_prefix")
     assert torch.equal(ko.cpu(), want[0]) and torch.equal(vo.cpu(), want[1])
     assert pad == 0 or all(torch.all(o[..., d:].cpu() == 7.0) for o in outs)
+
+
+@pytest.mark.parametrize("d,dtype,k,pad", [(128, torch.bfloat16, 1, 0), (128, torch.float16, 65, 0),
+                                           (64, torch.bfloat16, 257, 0), (64, torch.float16, 130, 4),
+                                           (128, torch.float32, 70, 0)])
+def test_gather_of_16_bit_rows(gpu, d, dtype, k, pad):
+    """Rows of a 16-bit prefix gathered in its own dtype (copied whole) and where their
+    strides allow no 16-byte loads (pad) or the dtype is f32; indices outside give zeros."""
+    g = torch.Generator().manual_seed(9)
+    n = 300
+    kf, vf = (torch.randn((2, 3, n, d + pad), generator=g).to(dtype) for _ in "kv")
+    idx = torch.randint(0, n, (2, 3, k), generator=g)
+    idx[0, 0, 0], idx[1, 2, -1] = -1, n
+    p = Prefix.dense(kf.to(gpu)[..., :d], vf.to(gpu)[..., :d])
+    ok, ov = gather_packed_kv(p, idx.to(gpu), dtype=dtype)
+    at = idx.clamp(0, n - 1).unsqueeze(-1).expand(-1, -1, -1, d)
+    dead = ((idx < 0) | (idx >= n)).unsqueeze(-1)
+    for got, src in ((ok, kf), (ov, vf)):
+        assert torch.equal(got.cpu(), torch.gather(src[..., :d], 2, at).masked_fill(dead, 0.0))
