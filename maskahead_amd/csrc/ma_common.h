@@ -125,7 +125,8 @@ enum { MA_DPP_SHL1 = 0x101, MA_DPP_SHL2 = 0x102, MA_DPP_SHL4 = 0x104, MA_DPP_SHL
        MA_DPP_SHR1 = 0x111, MA_DPP_SHR2 = 0x112, MA_DPP_SHR4 = 0x114, MA_DPP_SHR8 = 0x118,
        MA_DPP_BCAST15 = 0x142, MA_DPP_BCAST31 = 0x143 };
 
-// the value of another lane of the quad (CTRL: quad_perm; 0xB1 = lane ^ 1, 0x4E = lane ^ 2)
+// the value of another lane of the quad (CTRL quad_perm: 0xB1 = lane ^ 1, 0x4E = lane ^ 2), of 8
+// lanes (0x141 row_half_mirror: lane 7 - i) or of 16 (0x140 row_mirror: lane 15 - i)
 template <int CTRL>
 __device__ __forceinline__ float ma_quad(float x) {
     return __uint_as_float(ma_dpp<CTRL>(__float_as_uint(x)));

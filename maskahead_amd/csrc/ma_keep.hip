@@ -185,15 +185,19 @@ __global__ void __launch_bounds__(VS_NT) vs_partial_kernel(VsArgs a) {
 }
 
 // The all-bf16 form of the two passes (rows, 16-bit cache rows and vdtype bf16; bf16
-// mode): the same arithmetic as vs_partial_kernel / vs_score_kernel with every load of a
-// batch of VS_BATCH steps issued as straight-line code -- the slots (or rows) first, then
-// the codes, scales and 16-bit rows they name, at clamped addresses, the choices made by
-// selects afterwards -- so a thread has a batch's loads in flight together instead of
-// waiting for them one branch at a time.  HASQ / HASF: the cache lane has packed slots /
-// 16-bit rows (slot form; the dense form reads rows).
+// mode): the same results as vs_partial_kernel / vs_score_kernel with every load of a batch
+// of VS_BATCH steps issued as straight-line code -- the slots (or rows) first, then what they
+// name -- so a thread has a batch's loads in flight together instead of waiting for them one
+// branch at a time.  pw[u]: 8 channels of entry u as bf16 pairs, as the 16-bit rows hold them.
+// HASQ / HASF: the cache lane has packed slots / 16-bit rows (slot form; the dense form reads
+// rows).  A wave whose slots are all packed -- nearly every one: a cache's 16-bit rows are its
+// newest -- takes code words alone; another loads both at clamped addresses and selects.
+// (Bound by VALU work in the slot form: 112 lanes of 32 800 slots, D 128, 120.7 us for the
+// partial sums and 120.8 for the scores; 163.7 and 241.5 when every wave loaded both and
+// selected, and the scores were summed and rooted in f64.)
 template <bool SLOTS, bool HASQ, bool HASF>
 __device__ __forceinline__ void load_batch_bf(const VsArgs &a, int row, int jb, int j0, int j1, int tl, int c0,
-                                              float (&x)[VS_BATCH][8], float (&aw)[VS_BATCH]) {
+                                              uint32_t (&pw)[VS_BATCH][4], float (&aw)[VS_BATCH]) {
     const float *ar = a.a + (int64_t)row * a.sa;
     int jl[VS_BATCH];
 #pragma unroll
@@ -202,78 +206,76 @@ __device__ __forceinline__ void load_batch_bf(const VsArgs &a, int row, int jb, 
         jl[u] = j < j1 ? j : j0;
         aw[u] = ar[jl[u]];
     }
+    const int b = row / a.H, h = row % a.H;
+    auto put = [&](int u, const uint4 &r) {
+        pw[u][0] = r.x;
+        pw[u][1] = r.y;
+        pw[u][2] = r.z;
+        pw[u][3] = r.w;
+    };
     if constexpr (!SLOTS) {
-        uint4 w[VS_BATCH];
+        const uint16_t *v = (const uint16_t *)a.v + b * a.sv0 + h * a.sv1 + c0;
 #pragma unroll
-        for (int u = 0; u < VS_BATCH; ++u) w[u] = *(const uint4 *)((const uint16_t *)vrow(a, row, jl[u]) + c0);
-#pragma unroll
-        for (int u = 0; u < VS_BATCH; ++u) {
-            const uint32_t wv[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[u][i] = ma_bf16_to_f32((uint16_t)(wv[i >> 1] >> ((i & 1) * 16)));
-        }
+        for (int u = 0; u < VS_BATCH; ++u) put(u, *(const uint4 *)(v + (int64_t)jl[u] * a.sv2));
     } else {
-        const int b = row / a.H, h = row % a.H;
         int sl[VS_BATCH];
 #pragma unroll
         for (int u = 0; u < VS_BATCH; ++u) sl[u] = a.slots[(int64_t)row * a.sslot + jl[u]];
         const int cg = c0 / 32;
-        uint32_t w[VS_BATCH];
-        uint16_t scb[VS_BATCH], zeb[VS_BATCH];
-        uint4 r[VS_BATCH];
+        // (inner strides: the host has checked that they fit 32 bits)
+        const uint8_t *vq = a.vq + b * a.svq[0] + h * a.svq[1] + cg * a.svq[3] + (c0 % 32) / 2;
+        const int64_t so = b * a.svs[0] + h * a.svs[1] + cg;
+        const uint16_t *vf = (const uint16_t *)a.vf + b * a.svf[0] + h * a.svf[1] + c0;
+        const int q2 = (int)a.svq[2], s2 = (int)a.svs[2], f2 = (int)a.svf[2];
+        auto codes = [&](int u, uint32_t w, uint16_t scb, uint16_t zeb) {
+            const float sc = ma_f16_to_f32(scb), ze = ma_f16_to_f32(zeb);
+            uint32_t ev, od;   // codes of channels 0, 2, 4, 6 and 1, 3, 5, 7
+            ma_nibble_bytes(w, ev, od);
+            put(u, uint4{ma_pack_bf16x2(__builtin_fmaf(ma_ubyte_f32<0>(ev), sc, ze), __builtin_fmaf(ma_ubyte_f32<0>(od), sc, ze)),
+                         ma_pack_bf16x2(__builtin_fmaf(ma_ubyte_f32<1>(ev), sc, ze), __builtin_fmaf(ma_ubyte_f32<1>(od), sc, ze)),
+                         ma_pack_bf16x2(__builtin_fmaf(ma_ubyte_f32<2>(ev), sc, ze), __builtin_fmaf(ma_ubyte_f32<2>(od), sc, ze)),
+                         ma_pack_bf16x2(__builtin_fmaf(ma_ubyte_f32<3>(ev), sc, ze), __builtin_fmaf(ma_ubyte_f32<3>(od), sc, ze))});
+        };
+        if constexpr (HASQ) {
+            bool packed = true;
 #pragma unroll
-        for (int u = 0; u < VS_BATCH; ++u) {
-            const int s = sl[u];
-            if constexpr (HASQ) {
-                const int sq = s >= 0 && s < a.nq ? s : 0;
-                w[u] = *(const uint32_t *)(a.vq + b * a.svq[0] + h * a.svq[1] + (int64_t)sq * a.svq[2] +
-                                           cg * a.svq[3] + (c0 % 32) / 2);
-                const int64_t so = b * a.svs[0] + h * a.svs[1] + (int64_t)sq * a.svs[2] + cg;
-                scb[u] = a.vsc[so];
-                zeb[u] = a.vzp[so];
-            }
-            if constexpr (HASF) {
-                const int sf = s >= a.nq && s < a.nq + a.nf ? s - a.nq : 0;
-                r[u] = *(const uint4 *)((const uint16_t *)a.vf + b * a.svf[0] + h * a.svf[1] +
-                                        (int64_t)sf * a.svf[2] + c0);
+            for (int u = 0; u < VS_BATCH; ++u) packed = packed && (uint32_t)sl[u] < (uint32_t)a.nq;
+            if (__all(packed)) {
+                uint32_t w[VS_BATCH];
+                uint16_t scb[VS_BATCH], zeb[VS_BATCH];
+#pragma unroll
+                for (int u = 0; u < VS_BATCH; ++u) {
+                    w[u] = *(const uint32_t *)(vq + (int64_t)sl[u] * q2);
+                    scb[u] = a.vsc[so + (int64_t)sl[u] * s2];
+                    zeb[u] = a.vzp[so + (int64_t)sl[u] * s2];
+                }
+#pragma unroll
+                for (int u = 0; u < VS_BATCH; ++u) codes(u, w[u], scb[u], zeb[u]);
+                return;
             }
         }
 #pragma unroll
         for (int u = 0; u < VS_BATCH; ++u) {
             const int s = sl[u];
             const bool q = HASQ && s >= 0 && s < a.nq, f = HASF && s >= a.nq && s < a.nq + a.nf;
-            float sc = 0.f, ze = 0.f;
-            uint32_t wu = 0;
-            uint32_t rv[4] = {0u, 0u, 0u, 0u};
+            uint4 r = uint4{0u, 0u, 0u, 0u};
+            if constexpr (HASF) r = *(const uint4 *)(vf + (int64_t)(f ? s - a.nq : 0) * f2);
             if constexpr (HASQ) {
-                sc = ma_f16_to_f32(scb[u]);
-                ze = ma_f16_to_f32(zeb[u]);
-                wu = w[u];
+                const int sq = q ? s : 0;
+                codes(u, *(const uint32_t *)(vq + (int64_t)sq * q2), a.vsc[so + (int64_t)sq * s2],
+                      a.vzp[so + (int64_t)sq * s2]);
             }
-            if constexpr (HASF) {
-                rv[0] = r[u].x;
-                rv[1] = r[u].y;
-                rv[2] = r[u].z;
-                rv[3] = r[u].w;
-            }
-            // the choice made on bf16 pairs (channels 2 i2, 2 i2 + 1 in one word, as the 16-bit
-            // rows hold them): one select and one mask per two values
-            const uint32_t keep = (q || f) ? 0xffffffffu : 0u;
+            const uint32_t rv[4] = {r.x, r.y, r.z, r.w};
+            const uint32_t keep = (q || f) ? 0xffffffffu : 0u;   // a slot outside the cache is 0
 #pragma unroll
-            for (int i2 = 0; i2 < 4; ++i2) {
-                uint32_t pw = rv[i2];
-                if constexpr (HASQ) {
-                    const uint32_t pq = ma_pack_bf16x2(ma_dq((wu >> (8 * i2)) & 15u, sc, ze),
-                                                       ma_dq((wu >> (8 * i2 + 4)) & 15u, sc, ze));
-                    pw = q ? pq : pw;
-                }
-                pw &= keep;
-                x[u][2 * i2] = __uint_as_float(pw << 16);
-                x[u][2 * i2 + 1] = __uint_as_float(pw & 0xffff0000u);
-            }
+            for (int i = 0; i < 4; ++i) pw[u][i] = (HASQ && q ? pw[u][i] : rv[i]) & keep;
         }
     }
 }
+
+// the two channels of a bf16 pair
+__device__ __forceinline__ float pair_lo(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float pair_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
 template <bool SLOTS, bool HASQ, bool HASF>
 __global__ void __launch_bounds__(VS_NT) vs_partial_bf_kernel(VsArgs a) {
@@ -286,14 +288,18 @@ __global__ void __launch_bounds__(VS_NT) vs_partial_bf_kernel(VsArgs a) {
     double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     double den = 0.0;
     for (int jb = j0; jb < j1; jb += VS_TOK * VS_BATCH) {
-        float aw[VS_BATCH], x[VS_BATCH][8];
-        load_batch_bf<SLOTS, HASQ, HASF>(a, row, jb, j0, j1, tl, c0, x, aw);
+        float aw[VS_BATCH];
+        uint32_t pw[VS_BATCH][4];
+        load_batch_bf<SLOTS, HASQ, HASF>(a, row, jb, j0, j1, tl, c0, pw, aw);
 #pragma unroll
         for (int u = 0; u < VS_BATCH; ++u) {
             const bool ok = jb + u * VS_TOK + tl < j1;
             const double w = ok ? (double)ma_round_bf16(aw[u]) : 0.0;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[i] = __builtin_fma(w, (double)x[u][i], acc[i]);
+            for (int i = 0; i < 4; ++i) {
+                acc[2 * i] = __builtin_fma(w, (double)pair_lo(pw[u][i]), acc[2 * i]);
+                acc[2 * i + 1] = __builtin_fma(w, (double)pair_hi(pw[u][i]), acc[2 * i + 1]);
+            }
             den += w;
         }
     }
@@ -312,6 +318,15 @@ __global__ void __launch_bounds__(VS_NT) vs_partial_bf_kernel(VsArgs a) {
     }
 }
 
+// The score of an entry is a * bf16(sqrt(ss)), ss = the sum of the squared bf16 differences,
+// which the f64 sum of vs_score_kernel gives to well below an f32 ulp.  Here ss is summed in
+// f32 first: 8 products a lane in v_dot2 pairs and 4 lane exchanges, all terms positive, so
+// at most 12 roundings of 2^-23 (v_dot2 may truncate), half of that in the root, and an ulp
+// for v_sqrt: under 16 f32 ulps of the true root.  Unless the root lies within VS_NEAR ulps of
+// the middle between two bf16 values, its rounding to bf16 is therefore the f64 one's; the
+// others (about 1 entry in 500), and sums outside [1e-30, 1e30] (no f32 product of theirs has
+// under- or overflowed), are done again in f64.
+constexpr int VS_NEAR = 64;
 template <bool SLOTS, bool HASQ, bool HASF>
 __global__ void __launch_bounds__(VS_NT) vs_score_bf_kernel(VsArgs a) {
     __shared__ float cen[128];
@@ -327,22 +342,51 @@ __global__ void __launch_bounds__(VS_NT) vs_score_bf_kernel(VsArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) cc[i] = cen[c0 + i];
     for (int jb0 = j0; jb0 < j1; jb0 += VS_TOK * VS_BATCH) {
-        float x[VS_BATCH][8], aw[VS_BATCH];
-        load_batch_bf<SLOTS, HASQ, HASF>(a, row, jb0, j0, j1, tl, c0, x, aw);
+        float aw[VS_BATCH];
+        uint32_t pw[VS_BATCH][4];
+        load_batch_bf<SLOTS, HASQ, HASF>(a, row, jb0, j0, j1, tl, c0, pw, aw);
+        float mine = 0.f, weight = 0.f;   // lane oc of an entry's 16: step oc of the batch
 #pragma unroll
         for (int u = 0; u < VS_BATCH; ++u) {
-            const int j = jb0 + u * VS_TOK + tl;
+            float ss = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bf16x2_t d = __builtin_bit_cast(
+                    bf16x2_t, ma_pack_bf16x2(pair_lo(pw[u][i]) - cc[2 * i], pair_hi(pw[u][i]) - cc[2 * i + 1]));
+                ss = __builtin_amdgcn_fdot2_f32_bf16(d, d, ss, false);
+            }
+            if (!cok) ss = 0.f;
+            ss += ma_quad<0xB1>(ss);      // lanes ^ 1, then the other pair of the quad
+            ss += ma_quad<0x4E>(ss);
+            ss += ma_quad<0x141>(ss);     // the other quad of 8 lanes, then the other 8 of 16
+            ss += ma_quad<0x140>(ss);
+            mine = oc == u ? ss : mine;
+            weight = oc == u ? aw[u] : weight;
+        }
+        const uint32_t root = __float_as_uint(__builtin_amdgcn_sqrtf(mine));
+        const int j = jb0 + oc * VS_TOK + tl;
+        const bool own = oc < VS_BATCH && j < j1;
+        const bool decided = mine >= 1e-30f && mine <= 1e30f &&
+                             (uint32_t)((int)(root & 0xffffu) - 0x8000 + VS_NEAR) > 2u * VS_NEAR;
+        if (own && decided) sr[j] = weight * __uint_as_float((root + 0x8000u) & 0xffff0000u);
+        const uint64_t redo = __ballot(own && !decided);   // bit tl % 4 * 16 + u of this wave
+        if (redo == 0) continue;
+#pragma unroll
+        for (int u = 0; u < VS_BATCH; ++u) {
+            if (((redo >> u) & 0x0001000100010001ull) == 0) continue;
             double ss = 0.0;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float dl = ma_round_bf16(x[u][i] - cc[i]);
-                ss = __builtin_fma((double)dl, (double)dl, ss);
+            for (int i = 0; i < 4; ++i) {
+                const float d0 = ma_round_bf16(pair_lo(pw[u][i]) - cc[2 * i]);
+                const float d1 = ma_round_bf16(pair_hi(pw[u][i]) - cc[2 * i + 1]);
+                ss = __builtin_fma((double)d0, (double)d0, ss);
+                ss = __builtin_fma((double)d1, (double)d1, ss);
             }
             if (!cok) ss = 0.0;
             // sum over the 16 lanes of this entry (lanes tl*16 .. tl*16+15 of the wave pair)
 #pragma unroll
             for (int o = 8; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 16);
-            if (j < j1 && oc == 0) sr[j] = aw[u] * bf16_via_f32(__builtin_sqrt(ss));
+            if (own && !decided && oc == u) sr[j] = weight * bf16_via_f32(__builtin_sqrt(ss));
         }
     }
 }
@@ -663,7 +707,9 @@ extern "C" int ma_value_score_slots(const float *a, int64_t a_stride, const ma_p
     va.fdtype = p->fdtype;
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid(va.nchunks, rows);
-    if (vdtype == MA_BF16 && !fp32_mode && (p->nf == 0 || p->fdtype == MA_BF16)) {
+    auto fits = [](int64_t st) { return st >= INT32_MIN && st <= INT32_MAX; };
+    if (vdtype == MA_BF16 && !fp32_mode && (p->nf == 0 || p->fdtype == MA_BF16) && fits(p->svq[2]) && fits(p->svs[2]) &&
+        fits(p->svf[2])) {
         // the all-bf16 passes, instantiated for packed slots, 16-bit rows or both
         auto both = [&](auto partial, auto score) {
             hipLaunchKernelGGL(partial, grid, dim3(VS_NT), 0, st, va);
