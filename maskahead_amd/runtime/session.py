@@ -184,9 +184,9 @@ def lookahead_scores(cache, state, a1: dict, a_probe: dict | None = None, *, use
     if per_slot:
         a_all = a_all.gather(-1, state.phys[..., :live].to(torch.int64))
     if a_probe is not None:
-        for layer in range(L):
-            if layer in a_probe:
-                a_all[layer] += a_probe[layer]
+        probed = [layer for layer in range(L) if layer in a_probe]
+        if probed:    # every layer's sum in one launch
+            torch._foreach_add_([a_all[layer] for layer in probed], [a_probe[layer] for layer in probed])
     if not use_value:
         return a_all
     # value_score(a, live_values(cache, state, layer)) of every layer in one call, the layers
