@@ -185,6 +185,54 @@ struct FwdSmem {
         uint4 o[MAXS][4 * D];   // 32 x D f16 per row tile (write_partial)
     } u;
     uint64_t kmask[NBUF];
+    uint4 qx[MAXS - 4][4 * D];  // with the third K and V buffers: 32 x D bf16 per row tile (QRows)
+
+    // where wave w's query rows pass through (nothing of a tile is in the third buffers
+    // before the first barrier)
+    __device__ __forceinline__ uint4 *qrows(int w) {
+        static_assert(sizeof(KTileL<D>) >= 2 * 32 * D * 2 && sizeof(VTileL<D>) >= 2 * 32 * D * 2, "two row tiles each");
+        return w < 2 ? (uint4 *)u.t.kt[2].k + w * 4 * D : w < 4 ? (uint4 *)u.t.vt[2].vt + (w - 2) * 4 * D : qx[w - 4];
+    }
+};
+
+// The Q^T fragments of a row tile (lane: row c32, channels ks * 16 + hf * 8 .. + 7).  Loaded
+// as whole rows, D / 8 lanes a row, and turned in the wave's own LDS: fragments loaded
+// directly touch 32 bytes of each of 32 rows per instruction, and behind the 32 KB of a 16-bit
+// tile the last of them came ~2 000 cycles after the tile itself (8 000): a sub-step over
+// 2 048 entries 16.4 -> 15.9 us.  A packed tile is a third of that and its dequantization
+// covers the wait: there the turn through LDS only cost (544 tokens 40.9 -> 41.5 us a step).
+template <int D>
+struct QRows {
+    static constexpr int CH = D / 8, NI = 32 * CH / 64;
+    bf16x8_t raw[NI];
+
+    __device__ __forceinline__ void issue(const FwdArgs &a, int b, int h, int rtile, int lane) {
+        const int c32 = lane & 31, row = rtile * 32 + c32;
+        const bool ok = row < a.R;
+        const int g = ok ? row / a.T : 0, t = ok ? row % a.T : 0;
+        const int64_t off = (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2] + b * a.q.s[0];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {   // rows past R load row 0 (zeroed in finish)
+            const int r = i * (64 / CH) + lane / CH;
+            const int64_t ro = (int64_t)(uint32_t)__shfl((int)off, r) | ((int64_t)__shfl((int)(off >> 32), r) << 32);
+            raw[i] = ma_load8_as_bf16(a.q.ptr, ro + lane % CH * 8, a.q.dtype);
+        }
+    }
+    __device__ __forceinline__ void finish(const FwdArgs &a, int rtile, int lane, uint4 *lds, bf16x8_t *qf) {
+        const int c32 = lane & 31, hf = lane >> 5;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int r = i * (64 / CH) + lane / CH;
+            lds[r * CH + (lane % CH ^ r % CH)] =
+                rtile * 32 + r < a.R ? __builtin_bit_cast(uint4, raw[i]) : uint4{0u, 0u, 0u, 0u};
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks)
+            qf[ks] = __builtin_bit_cast(bf16x8_t, lds[c32 * CH + ((2 * ks + hf) ^ c32 % CH)]);
+    }
 };
 
 // s_softmax with the probabilities kept in registers: pb[c] = P^T chunk c (16 tokens) in
@@ -667,18 +715,27 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
     // prologue: tiles 0 and 1 staged, tile 2's loads in flight; Q of the row tile
     if (nt > 0) load_tile(0);
     bf16x8_t qf[NKS];
-    if (is_s) {
-        const int g = row_ok ? row / a.T : 0, t = row_ok ? row % a.T : 0;
-        const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
+    if constexpr (SRC == 0) {
+        if (is_s) {
+            const int g = row_ok ? row / a.T : 0, t = row_ok ? row % a.T : 0;
+            const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) qf[ks] = ma_load8_as_bf16(a.q.ptr, qb + ks * 16 + hf * 8, a.q.dtype);
+            for (int ks = 0; ks < NKS; ++ks) qf[ks] = ma_load8_as_bf16(a.q.ptr, qb + ks * 16 + hf * 8, a.q.dtype);
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) qf[ks] = row_ok ? qf[ks] : bf16x8_t{};
-    }
-    if (nt > 0) store_tile(0);
-    if (nt > 1) {
-        load_tile(1);
-        store_tile(1);
+            for (int ks = 0; ks < NKS; ++ks) qf[ks] = row_ok ? qf[ks] : bf16x8_t{};
+        }
+        if (nt > 0) store_tile(0);
+        if (nt > 1) {
+            load_tile(1);
+            store_tile(1);
+        }
+    } else {
+        QRows<D> qr;
+        if (is_s) qr.issue(a, b, h, rtile, lane);
+        if (nt > 0) store_tile(0);
+        if (nt > 1) load_tile(1);
+        if (is_s) qr.finish(a, rtile, lane, S.qrows(wave), qf);
+        if (nt > 1) store_tile(1);
     }
     if (nt > 2) load_tile(2);
     __syncthreads();
