@@ -925,6 +925,87 @@ __global__ void __launch_bounds__(128) splitk_combine_kernel(FwdArgs a, ma_tenso
     }
 }
 
+// Pass 2 for at most CMB_FEW splits and many rows (a prefill chunk: 3 584 rows of 4 splits).
+// splitk_combine_kernel spends a 128-thread workgroup and two barriers on each row; here a
+// thread merges 8 channels of a row over all of its splits by itself, 16 rows of D 128 to a
+// workgroup, every load in flight at once and no barrier.  Bound by bytes: 14 336 rows, 38 MB,
+// 34.3 us a workgroup per row, 8.1 so.
+constexpr int CMB_FEW = 8, CMB_NT = 256;
+template <int D>
+__global__ void __launch_bounds__(CMB_NT) splitk_combine_few_kernel(FwdArgs a, ma_tensor4 out, float *mp_out,
+                                                                    float *lp_out, void *op_out, int vec) {
+    constexpr int OCT = D / 8, ROWS = CMB_NT / OCT;
+    typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
+    const int bh = blockIdx.x % a.BH, b = bh / a.H, h = bh % a.H;   // lane-fastest, as pass 1
+    const int row = blockIdx.x / a.BH * ROWS + threadIdx.x / OCT, oc = threadIdx.x % OCT;
+    if (row >= a.R) return;
+    const int R = a.R, nsplit = a.nsplit;
+    const int64_t base = (int64_t)bh * (nsplit + 1) * R + row;
+    // slots 0 .. nsplit - 1 are the prefix's, slot nsplit the current block's
+    float m[CMB_FEW + 1], l[CMB_FEW + 1], sc[CMB_FEW + 1];
+    f16x8_t o[CMB_FEW + 1];
+#pragma unroll
+    for (int i = 0; i <= CMB_FEW; ++i) {
+        const int64_t pr = base + (int64_t)min(i, nsplit) * R;
+        m[i] = a.wm[pr];
+        l[i] = a.wl[pr];
+        sc[i] = a.wsc[pr];
+        o[i] = *(const f16x8_t *)&a.wo[pr * D + oc * 8];
+    }
+    float M = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < CMB_FEW; ++i) M = i < nsplit ? fmaxf(M, m[i]) : M;
+    const float msafe = M == -INFINITY ? 0.f : M;
+    float op[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float lp = 0.f;
+#pragma unroll
+    for (int i = 0; i < CMB_FEW; ++i) {
+        const float w = l[i] * expf(m[i] - msafe);
+        if (i < nsplit && w != 0.f) {   // an empty split (weight 0) adds nothing
+            const float ws = w * sc[i];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) op[e] = __builtin_fmaf(ws, (float)o[i][e], op[e]);
+            lp += w;
+        }
+    }
+    // loads past nsplit repeated the current block's slot, so the last one is it
+    const float mc = m[CMB_FEW], lc = l[CMB_FEW], scc = lc > 0.f ? sc[CMB_FEW] : 0.f;
+    const float mm = fmaxf(M, mc), ms = mm == -INFINITY ? 0.f : mm;
+    const float ea = expf(M - ms), eb = expf(mc - ms);
+    const float den = lp * ea + lc * eb;
+    const float inv = 1.0f / (den > 0.f ? den : 1.0f), invp = 1.0f / (lp > 0.f ? lp : 1.0f);
+    float y[8], yp[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float oc_d = lc > 0.f ? (float)o[CMB_FEW][e] * scc : 0.f;
+        y[e] = (op[e] * ea + lc * oc_d * eb) * inv;
+        yp[e] = op[e] * invp;
+    }
+    const int g = row / a.T, t = row % a.T;
+    auto put = [&](void *p, int64_t off, const float (&x)[8], bool v16) {
+        if (v16) {
+            uint32_t w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                w[e] = out.dtype == MA_BF16 ? ma_pack_bf16x2(x[2 * e], x[2 * e + 1])
+                                            : (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x[2 * e]) |
+                                                  ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x[2 * e + 1]) << 16);
+            *(uint4 *)((uint16_t *)p + off) = uint4{w[0], w[1], w[2], w[3]};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ma_store_f(p, off + e, out.dtype, x[e]);
+        }
+    };
+    put(out.ptr, b * out.s[0] + (int64_t)(h * a.G + g) * out.s[1] + (int64_t)t * out.s[2] + oc * 8, y, vec & 1);
+    if (mp_out) {
+        if (oc == 0) {
+            mp_out[(int64_t)bh * R + row] = M;
+            lp_out[(int64_t)bh * R + row] = lp;
+        }
+        put(op_out, ((int64_t)bh * R + row) * D + oc * 8, yp, vec & 2);
+    }
+}
+
 // The parts of a prefix: packed whole tiles [0, nq64) in splits, then -- packed prefixes --
 // the tail [nq64, tail_end), then the 16-bit part [tail_end, n) in splits of its own.  The
 // residual of a cache (fewer than 64 tokens, unless blocks are staged unquantized) joins the
@@ -1127,6 +1208,19 @@ int launch_merge(const Plan &pl, ma_tensor4 out, float *mp, float *lp, void *op,
         return MA_EINVAL;
     }
     const FwdArgs &fa = pl.fa;
+    if (fa.nsplit <= CMB_FEW) {
+        const int rows = CMB_NT / (pl.D / 8);
+        const dim3 fgrid((fa.R + rows - 1) / rows * fa.BH);
+        // 16-byte stores of 16-bit outputs whose rows allow them (bit 0 out, bit 1 op)
+        const bool b16 = out.dtype != MA_F32;
+        const int vec = (b16 && aligned16(out.ptr) && out.s[0] % 8 == 0 && out.s[1] % 8 == 0 && out.s[2] % 8 == 0 ? 1 : 0) |
+                        (b16 && aligned16(op) ? 2 : 0);
+        if (pl.D == 128)
+            hipLaunchKernelGGL(splitk_combine_few_kernel<128>, fgrid, dim3(CMB_NT), 0, st, fa, out, mp, lp, op, vec);
+        else
+            hipLaunchKernelGGL(splitk_combine_few_kernel<64>, fgrid, dim3(CMB_NT), 0, st, fa, out, mp, lp, op, vec);
+        return ma_check_launch("ma_splitk_merge");
+    }
     const dim3 cgrid(fa.R * pl.B * fa.H);
     if (pl.D == 128)
         hipLaunchKernelGGL(splitk_combine_kernel<128>, cgrid, dim3(128), 0, st, fa, out, mp, lp, op);
