@@ -27,6 +27,7 @@
 // load per row) and the value centre (mean of O_p over the selection rows, a fixed-order
 // LDS reduction shared with ma_value_centre).
 #include <atomic>
+#include <type_traits>
 
 #include "ma_stage.h"
 
@@ -42,16 +43,13 @@ enum { SRC_PACKED = 0, SRC_DENSE = 1 };
 struct ScoreArgs {
     ma_tensor4 q;
     PrefixDev pre;
-    const int32_t *q_rows;   // NULL: the selection rows are block positions row0 .. row0 + T2 - 1
-    int row0;
+    const int32_t *q_rows;   // NULL: the selection rows are block positions 0 .. T2 - 1
     const float *mp, *lp;
     const void *op;  // prefix-only output [B*H, R, D] (op_dtype): the value centre's source
     int op_dtype;
     float *mass, *score;
     int H, G, T, T2, R, R2, row_tiles, value;
     int vround;    // 0, or MA_BF16 / MA_F16: packed values rounded to that dtype for the distance
-    int r2_total;  // selection rows of the whole call (the mean's divisor) when rows run in passes
-    int accum;     // this pass adds its share to mass (passes after the first; mass only)
     int nfast;     // whole tiles of the source kind per lane: tiles [0, nfast)
     int per;       // tiles per fast workgroup
     int fast_wgs;  // fast workgroups per lane (blockIdx.x below it); then one tail tile each
@@ -446,7 +444,7 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
     };
     // selection row rr = g * T2 + i: block position t (clamped into the block), row g * T + t
     auto sel_pos = [&](int rr, int g) {
-        return min(max(ident ? a.row0 + rr - g * T2 : sm.qr[rr - g * T2], 0), T - 1);
+        return min(max(ident ? rr - g * T2 : sm.qr[rr - g * T2], 0), T - 1);
     };
     const int rt_pad = 32 * row_tiles;
     // Q of the unit's row tile: in-order rows need no table, so their loads are issued
@@ -544,8 +542,7 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
 #pragma unroll
             for (int j = 0; j < CB; ++j) {
                 const int r = r0 + j * CS;
-                const int tpos = r % T - a.row0;
-                wgt[j] = r >= R ? 0.f : ident ? (tpos >= 0 && tpos < T2 ? 1.f : 0.f) : (float)sm.cnt[r];
+                wgt[j] = r >= R ? 0.f : ident ? (r % T < T2 ? 1.f : 0.f) : (float)sm.cnt[r];
             }
             if (a.op_dtype == MA_F32) {
                 // f32 rows: 8 channels in two 16-byte halves
@@ -625,7 +622,7 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
         }
     };
 
-    const float inv_r2 = 1.0f / (float)a.r2_total;
+    const float inv_r2 = 1.0f / (float)R2;
     const int hist_rank = HIST ? a.hist_rank : 0;   // HIST: 1 or 2
     auto finish = [&](int tile, int rb, int db) {
         const int j = tile * TILE + lane;
@@ -644,15 +641,14 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
             const int64_t o = (int64_t)bh * end + j;
             if (a.pre.mask) live = a.pre.mask[o] != 0;
             const float m = live ? s * inv_r2 : 0.f;
-            const float mf = a.accum ? a.mass[o] + m : m;   // the mass after this pass
-            a.mass[o] = mf;
+            a.mass[o] = m;
             float sc = 0.f;
             if (value) {
                 sc = live ? m * __builtin_sqrtf(sm.dist[db][lane]) : 0.f;
                 a.score[o] = sc;
             }
             // the key ma_topk_select gives this slot under the same mask
-            if constexpr (HIST) key = ma_order_key(live ? (hist_rank == 2 ? sc : mf) : -__builtin_inff());
+            if constexpr (HIST) key = ma_order_key(live ? (hist_rank == 2 ? sc : m) : -__builtin_inff());
         }
         if constexpr (HIST) {
             const int r = tile - tile0;   // tile of the run
@@ -913,7 +909,7 @@ __device__ __forceinline__ void small_units(const ScoreArgs &a, SmallSmem<D> &sm
     float *dist = sm.dist[wave];
     const bool value = a.value;
     const int vround = a.vround;
-    const float inv_r2 = 1.0f / (float)a.r2_total, sl2 = a.sl2;
+    const float inv_r2 = 1.0f / (float)a.R2, sl2 = a.sl2;
     if (!loaded) {
         small_offsets<D, KIND>(L, W);
         small_load<D, KIND>(L, W, u0, end, value);
@@ -1024,7 +1020,7 @@ __global__ void __launch_bounds__(SM_NT) score_small_kernel(ScoreArgs a, int uni
     auto sel = [&](int rr, int &g, int &t) {
         g = rr / T2;
         const int i = rr - g * T2;
-        t = min(max(ident ? a.row0 + i : a.q_rows[i], 0), T - 1);
+        t = min(max(ident ? i : a.q_rows[i], 0), T - 1);
     };
     for (int e = tid; e < ROWS * (D / 8); e += SM_NT) {
         const int rr = e / (D / 8), c = e % (D / 8);
@@ -1068,6 +1064,165 @@ __global__ void __launch_bounds__(SM_NT) score_small_kernel(ScoreArgs a, int uni
     if (has_t) {
         if (dense_vec) small_units<D, 1, ROWS>(a, sm, L, W, bh, wave, ts, u1, end, !has_p);
         else small_units<D, 2, ROWS>(a, sm, L, W, bh, wave, ts, u1, end, false);
+    }
+}
+
+// ------------------------------------------------------------------ many selection rows
+// The mass of more selection rows than score_kernel's 16 waves hold (a prefill chunk's: G x
+// 512).  Split by tokens: a workgroup of 8 waves dequantizes MS_TILES tiles into LDS once and
+// meets again only to add the waves' sums.  Between, every wave takes pairs of row tiles (64
+// rows, Q in registers) over all of the workgroup's tokens: a K fragment read from LDS
+// serves two MFMAs, and the MFMAs of the next 32 tokens are issued between the exp2 of
+// these.  Bound by MFMA and exp2 issue.  (In passes of 512 rows, each a launch that staged
+// every tile again, a 512-token chunk of 7 heads over 16 384 tokens took 8 x 17.5 us.)
+constexpr int MS_NT = 512, MS_WAVES = MS_NT / 64, MS_TILES = 7;
+
+template <int D>
+struct MassSmem {
+    KTileL<D> kt[MS_TILES];
+    float sum[MS_WAVES][MS_TILES * TILE];
+    float crow[MS_WAVES][64];
+};
+
+template <int D>
+__global__ void __launch_bounds__(MS_NT) mass_rows_kernel(ScoreArgs a, int items_ok) {
+    __shared__ MassSmem<D> sm;
+    constexpr int KS = D + 8, NKS = D / 16, NIK = 4 * D;   // items of a tile: 8 tokens x 2 channels, or 16 channels
+    constexpr int NIT = (MS_TILES * NIK + MS_NT - 1) / MS_NT;
+    const int h = blockIdx.y, b = blockIdx.z, bh = b * a.H + h;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c32 = lane & 31, hf = lane >> 5;
+    const int nq = a.pre.nq, end = nq + a.pre.nf;
+    const int tile0 = blockIdx.x * a.per, n0 = tile0 * TILE;
+    const int nt = min(a.per, (end + TILE - 1) / TILE - tile0);
+    const Lane L = make_lane(a.pre, b, h, bh);
+    if (items_ok) {
+        // an item's 32-token half is packed, or 16-bit rows (those past the end repeat the last)
+        uint32_t w[NIT][8];
+#pragma unroll
+        for (int r = 0; r < NIT; ++r) {
+            const int it = tid + r * MS_NT, ti = it / NIK, u = it % NIK;
+            const int t0 = n0 + ti * TILE;
+            if (ti >= nt) continue;
+            if (t0 + u / (2 * D) * KGRP < nq) {
+                const int64_t g = t0 / KGRP;
+                kp_load(w[r], L.kq + g * L.kq_g, L.ks + g * L.ks_g, L.kz + g * L.ks_g, L.kq_d, kp_offsets<D>(L, u));
+            } else if (a.pre.nf > 0) {
+                const int64_t row = min(t0 + u / (D / 16), end - 1) - nq;
+                d32_load(w[r], L.kf + (row * L.kf_n + u % (D / 16) * 16) * 2, 0u);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < NIT; ++r) {
+            const int it = tid + r * MS_NT, ti = it / NIK, u = it % NIK;
+            if (ti >= nt) continue;
+            if (n0 + ti * TILE + u / (2 * D) * KGRP < nq) kp_store<D>(sm.kt[ti].k, w[r], u);
+            else if (a.pre.nf > 0) kd_store<D>(sm.kt[ti].k, w[r], u, a.pre.fdtype);
+        }
+    } else {
+#pragma unroll 1
+        for (int it = tid; it < nt * TILE * D; it += MS_NT) {
+            const int t = it / D, d = it % D;
+            sm.kt[t / TILE].k[t % TILE * KS + d] = ma_f32_to_bf16(n0 + t < end ? lane_key(L, n0 + t, d) : 0.f);
+        }
+    }
+    for (int i = lane; i < MS_TILES * TILE; i += 64) sm.sum[wave][i] = 0.f;
+    __syncthreads();
+
+    // pairs p = wave / share, ... of row tiles; with fewer pairs than waves `share` waves take a
+    // pair, each every share-th 32-token unit
+    const int T = a.T, T2 = a.T2, R2 = a.R2, R = a.R;
+    const int npair = (R2 + 63) / 64;
+    const int share = npair >= MS_WAVES ? 1 : npair >= 3 ? 2 : npair == 2 ? 4 : 8;
+    const int units = 2 * nt;
+    const float sl2 = a.sl2;
+    float *sum = sm.sum[wave], *crow = sm.crow[wave];
+    for (int p = wave / share; p < npair; p += MS_WAVES / share) {
+        bf16x8_t qf[2][NKS];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            // selection row rr = g * T2 + i: block position t (clamped into the block), row g * T + t
+            const int rr = p * 64 + e * 32 + c32, g = rr < R2 ? rr / T2 : 0, i = rr < R2 ? rr - g * T2 : 0;
+            const int t = min(max(a.q_rows ? a.q_rows[i] : i, 0), T - 1);
+            const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) qf[e][ks] = ma_load8_as_bf16(a.q.ptr, qb + ks * 16 + hf * 8, a.q.dtype);
+            // rows without a live prefix entry and padding rows add exactly 0
+            const float m = a.mp[(int64_t)bh * R + g * T + t], l = a.lp[(int64_t)bh * R + g * T + t];
+            const float c = rr < R2 && l > 0.f ? __builtin_fmaf(m, MA_LOG2E, __log2f(l)) : __builtin_inff();
+            if (hf == 0) crow[e * 32 + c32] = c;
+            if (rr >= R2) {
+#pragma unroll
+                for (int ks = 0; ks < NKS; ++ks) qf[e][ks] = bf16x8_t{};
+            }
+        }
+        wave_lds_sync();
+        f32x4_t c4[2][4];   // rows 8 * i4 + 4 * hf + 0..3 of each row tile
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) c4[e][i4] = *(const f32x4_t *)&crow[e * 32 + i4 * 8 + hf * 4];
+        wave_lds_sync();
+        // S of unit un into sn (when NEXT), between its MFMAs the exp2 of unit u's S (sc) and
+        // their sum over this wave's 64 rows
+        auto body = [&](int u, int un, f32x16_t *sc, f32x16_t *sn, auto next, auto cur) {
+            constexpr bool NEXT = decltype(next)::value, CUR = decltype(cur)::value;
+            const uint16_t *kr = &sm.kt[un >> 1].k[((un & 1) * 32 + c32) * KS + hf * 8];
+            float acc[2] = {0.f, 0.f};
+            auto expo = [&](int e, int i0) {
+#pragma unroll
+                for (int i = i0; i < i0 + 16 / NKS; ++i)
+                    acc[e] += __builtin_amdgcn_exp2f(__builtin_fmaf(sc[e][i], sl2, -c4[e][i >> 2][i & 3]));
+            };
+            if constexpr (NEXT) {
+                sn[0] = f32x16_t{};
+                sn[1] = f32x16_t{};
+            }
+            bf16x8_t kf, nkf;   // a fragment is read one k-step ahead
+            if constexpr (NEXT) nkf = *(const bf16x8_t *)kr;
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                if constexpr (NEXT) {
+                    kf = nkf;
+                    if (ks + 1 < NKS) nkf = *(const bf16x8_t *)(kr + (ks + 1) * 16);
+                    sn[0] = ma_mfma32(qf[0][ks], kf, sn[0]);
+                }
+                if constexpr (CUR) expo(0, ks * (16 / NKS));
+                if constexpr (NEXT && CUR) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (NEXT) sn[1] = ma_mfma32(qf[1][ks], kf, sn[1]);
+                if constexpr (CUR) expo(1, ks * (16 / NKS));
+                if constexpr (NEXT && CUR) __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (CUR) {
+                const float x = ma_sum_xor32(acc[0] + acc[1]);
+                if (hf == 0) sum[u * 32 + c32] += x;
+            }
+        };
+        constexpr std::true_type yes{};
+        constexpr std::false_type no{};
+        f32x16_t sa[2], sb[2];
+        int u = wave % share;
+        if (u < units) body(0, u, sb, sa, yes, no);
+        for (; u + 2 * share < units; u += 2 * share) {
+            body(u, u + share, sa, sb, yes, yes);
+            body(u + share, u + 2 * share, sb, sa, yes, yes);
+        }
+        if (u + share < units) {
+            body(u, u + share, sa, sb, yes, yes);
+            body(u + share, 0, sb, sa, no, yes);
+        } else if (u < units) {
+            body(u, 0, sa, sb, no, yes);
+        }
+    }
+    __syncthreads();
+    const float inv = 1.0f / (float)R2;
+    for (int i = tid; i < nt * TILE; i += MS_NT) {
+        const int j = n0 + i;
+        if (j >= end) break;
+        float x = 0.f;
+#pragma unroll
+        for (int w = 0; w < MS_WAVES; ++w) x += sm.sum[w][i];
+        const int64_t o = (int64_t)bh * end + j;
+        a.mass[o] = !a.pre.mask || a.pre.mask[o] != 0 ? x * inv : 0.f;
     }
 }
 
@@ -1179,9 +1334,6 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
         ma_set_error("%s: %d query heads per KV head exceed the built maximum %d", who, G, MAX_R2);
         return MA_EUNSUPPORTED;
     }
-    // mass only: the selection rows in passes of at most MAX_R2 rows (whole q_rows entries),
-    // each adding its share of the mean to mass
-    const int t2_pass = value ? T2 : (MAX_R2 / G < T2 ? MAX_R2 / G : T2);
     const int n = p->nq + p->nf;
     if (n == 0) return MA_OK;
     // 16-bit parts are read with 32-byte vector loads: every token row must stay aligned
@@ -1189,12 +1341,12 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
                                              ((uintptr_t)p->kf & 15) == 0 && ((uintptr_t)p->vf & 15) == 0 &&
                                              p->skf[0] % 16 == 0 && p->skf[1] % 16 == 0 && p->svf[0] % 16 == 0 &&
                                              p->svf[1] % 16 == 0);
-    const int row_tiles_max = (G * t2_pass + 31) / 32;
+    const int row_tiles = (R2 + 31) / 32;
     // one 1024-thread workgroup per CU: units of half a tile up to 8 row tiles, whole
     // tiles beyond.  (Two 512-thread workgroups per CU, NT = 512, measured 1.6x slower at
     // config 2: each workgroup loads its lane's Q and O_p rows in its prologue, so twice
     // the workgroups move twice those bytes.)
-    const int halves = row_tiles_max <= 8 ? 1 : 2;
+    const int halves = row_tiles <= 8 ? 1 : 2;
     const int wgs_per_cu = 1;
     const int tiles = (n + TILE - 1) / TILE;
     const bool packed = p->nq > 0;
@@ -1226,7 +1378,9 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
     sa.G = G;
     sa.T = T;
     sa.R = R;
-    sa.r2_total = R2;
+    sa.T2 = T2;
+    sa.R2 = R2;
+    sa.row_tiles = row_tiles;
     sa.value = value;
     if (v_round != 0 && v_round != MA_BF16 && v_round != MA_F16) {
         ma_set_error("%s: v_round must be 0, MA_BF16 or MA_F16", who);
@@ -1258,12 +1412,7 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
         const int waves_bh = max(1, min(units, 8 * ma_num_cus() / (B * H)));
         const int per = (units + waves_bh - 1) / waves_bh;
         const int waves = (units + per - 1) / per;
-        sa.q_rows = q_rows;
-        sa.row0 = 0;
-        sa.T2 = T2;
-        sa.R2 = R2;
         sa.row_tiles = 1;
-        sa.accum = 0;
         sa.per = per;
         const dim3 g2((waves + SM_WAVES - 1) / SM_WAVES, B * H);
         const int dv = dense_vec_ok ? 1 : 0;
@@ -1283,6 +1432,20 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
         // this pass does not build the histogram in-kernel: the select's own level-0 launch
         return ma_topk_level0_into_state(hist_rank == 2 ? score : mass, n, p->mask, n, B * H, n, topk_state, stream);
     }
+    // more rows than the 16 waves of score_kernel hold (mass only, checked above)
+    if (R2 > MAX_R2) {
+        // runs of at most MS_TILES tiles, as equal as whole dispatch waves allow
+        const int all = (tiles * B * H + ma_num_cus() - 1) / ma_num_cus();
+        const int waves = (all + MS_TILES - 1) / MS_TILES;
+        sa.per = (all + waves - 1) / waves;
+        const dim3 mgrid((tiles + sa.per - 1) / sa.per, H, B);
+        const int items = dense_vec_ok ? 1 : 0;
+        if (D == 128) hipLaunchKernelGGL(mass_rows_kernel<128>, mgrid, dim3(MS_NT), 0, st, sa, items);
+        else hipLaunchKernelGGL(mass_rows_kernel<64>, mgrid, dim3(MS_NT), 0, st, sa, items);
+        rc = ma_check_launch(who);
+        if (rc || !hist_rank) return rc;
+        return ma_topk_level0_into_state(mass, n, p->mask, n, B * H, n, topk_state, stream);
+    }
     sa.nfast = nfast;
     sa.tail_vec = packed && dense_vec_ok;
     sa.per = per;
@@ -1299,25 +1462,16 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
         if (halves == 1) MA_SCORE(D_, S_, 1);     \
         else MA_SCORE(D_, S_, 2);                 \
     } while (0)
-    for (int t0 = 0; t0 < T2; t0 += t2_pass) {
-        const int t2 = T2 - t0 < t2_pass ? T2 - t0 : t2_pass;
-        sa.q_rows = q_rows ? q_rows + t0 : nullptr;
-        sa.row0 = t0;
-        sa.T2 = t2;
-        sa.R2 = G * t2;
-        sa.row_tiles = (G * t2 + 31) / 32;
-        sa.accum = t0 > 0;
-        sa.hist_rank = t0 + t2 >= T2 ? hist_rank : 0;   // the last pass sees the final mass
-        if (D == 128) {
-            if (packed) MA_SCORE_I(128, SRC_PACKED);
-            else MA_SCORE_I(128, SRC_DENSE);
-        } else {
-            if (packed) MA_SCORE_I(64, SRC_PACKED);
-            else MA_SCORE_I(64, SRC_DENSE);
-        }
-        const int rc2 = ma_check_launch(who);
-        if (rc2) return rc2;
+    sa.hist_rank = hist_rank;
+    if (D == 128) {
+        if (packed) MA_SCORE_I(128, SRC_PACKED);
+        else MA_SCORE_I(128, SRC_DENSE);
+    } else {
+        if (packed) MA_SCORE_I(64, SRC_PACKED);
+        else MA_SCORE_I(64, SRC_DENSE);
     }
+    rc = ma_check_launch(who);
+    if (rc) return rc;
 #undef MA_SCORE_I
 #undef MA_SCORE
     // lanes beyond 31-bit offsets run the kernel without the in-kernel histogram
