@@ -77,6 +77,23 @@ __device__ __forceinline__ bf16x8_t ma_load8_as_bf16(const void *base, int64_t o
     return r;
 }
 
+// N such octets, at elements off(0) .. off(N - 1), into r[0 .. N - 1]: the dtype is looked at
+// once (asked per octet it cost five branches each, and the octets' loads were issued that
+// far apart)
+template <int N, class F>
+__device__ __forceinline__ void ma_load8n_as_bf16(const void *base, int dtype, F off, bf16x8_t *r) {
+    if (dtype == MA_BF16) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = *(const bf16x8_t *)((const uint16_t *)base + off(i));
+    } else if (dtype == MA_F16) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = ma_load8_as_bf16(base, off(i), MA_F16);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = ma_load8_as_bf16(base, off(i), MA_F32);
+    }
+}
+
 // x = f32(code) * f32(scale) + f32(zero); the product is exact, so fused or not the
 // result carries one rounding -- bit-identical to the reference's two torch ops.
 __device__ __forceinline__ float ma_dq(uint32_t code, float scale, float zero) {

@@ -457,8 +457,7 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
     auto load_q = [&](int qo) {
         const int64_t qb = b * a.q.s[0] + (int64_t)h * a.G * a.q.s[1] + (qo < 0 ? 0 : qo);
         const int ks0 = HALVES == 1 ? th0 * QH : 0;
-#pragma unroll
-        for (int j = 0; j < QH; ++j) qf[j] = ma_load8_as_bf16(a.q.ptr, qb + (ks0 + j) * 16 + hf * 8, a.q.dtype);
+        ma_load8n_as_bf16<QH>(a.q.ptr, a.q.dtype, [&](int j) { return qb + (ks0 + j) * 16 + hf * 8; }, qf);
     };
     if (s_wave && ident) {
         const int rr = rt * 32 + c32, g = rr / T2;
@@ -1144,8 +1143,7 @@ __global__ void __launch_bounds__(MS_NT) mass_rows_kernel(ScoreArgs a, int items
             const int rr = p * 64 + e * 32 + c32, g = rr < R2 ? rr / T2 : 0, i = rr < R2 ? rr - g * T2 : 0;
             const int t = min(max(a.q_rows ? a.q_rows[i] : i, 0), T - 1);
             const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) qf[e][ks] = ma_load8_as_bf16(a.q.ptr, qb + ks * 16 + hf * 8, a.q.dtype);
+            ma_load8n_as_bf16<NKS>(a.q.ptr, a.q.dtype, [&](int ks) { return qb + ks * 16 + hf * 8; }, qf[e]);
             // rows without a live prefix entry and padding rows add exactly 0
             const float m = a.mp[(int64_t)bh * R + g * T + t], l = a.lp[(int64_t)bh * R + g * T + t];
             const float c = rr < R2 && l > 0.f ? __builtin_fmaf(m, MA_LOG2E, __log2f(l)) : __builtin_inff();

@@ -211,12 +211,13 @@ struct QRows {
         const bool ok = row < a.R;
         const int g = ok ? row / a.T : 0, t = ok ? row % a.T : 0;
         const int64_t off = (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2] + b * a.q.s[0];
+        int64_t ro[NI];
 #pragma unroll
         for (int i = 0; i < NI; ++i) {   // rows past R load row 0 (zeroed in finish)
             const int r = i * (64 / CH) + lane / CH;
-            const int64_t ro = (int64_t)(uint32_t)__shfl((int)off, r) | ((int64_t)__shfl((int)(off >> 32), r) << 32);
-            raw[i] = ma_load8_as_bf16(a.q.ptr, ro + lane % CH * 8, a.q.dtype);
+            ro[i] = (int64_t)(uint32_t)__shfl((int)off, r) | ((int64_t)__shfl((int)(off >> 32), r) << 32);
         }
+        ma_load8n_as_bf16<NI>(a.q.ptr, a.q.dtype, [&](int i) { return ro[i] + lane % CH * 8; }, raw);
     }
     __device__ __forceinline__ void finish(const FwdArgs &a, int rtile, int lane, uint4 *lds, bf16x8_t *qf) {
         const int c32 = lane & 31, hf = lane >> 5;
@@ -408,8 +409,7 @@ __device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, 
     if (is_s) {
         const int g = row_ok ? row / a.T : 0, t = row_ok ? row % a.T : 0;
         const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) qf[ks] = ma_load8_as_bf16(a.q.ptr, qb + ks * 16 + hf * 8, a.q.dtype);
+        ma_load8n_as_bf16<NKS>(a.q.ptr, a.q.dtype, [&](int ks) { return qb + ks * 16 + hf * 8; }, qf);
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) qf[ks] = row_ok ? qf[ks] : bf16x8_t{};
     }
@@ -719,8 +719,7 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
         if (is_s) {
             const int g = row_ok ? row / a.T : 0, t = row_ok ? row % a.T : 0;
             const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) qf[ks] = ma_load8_as_bf16(a.q.ptr, qb + ks * 16 + hf * 8, a.q.dtype);
+            ma_load8n_as_bf16<NKS>(a.q.ptr, a.q.dtype, [&](int ks) { return qb + ks * 16 + hf * 8; }, qf);
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) qf[ks] = row_ok ? qf[ks] : bf16x8_t{};
         }
