@@ -1072,8 +1072,9 @@ __global__ void __launch_bounds__(SM_NT) score_small_kernel(ScoreArgs a, int uni
 // meets again only to add the waves' sums.  Between, every wave takes pairs of row tiles (64
 // rows, Q in registers) over all of the workgroup's tokens: a K fragment read from LDS
 // serves two MFMAs, and the MFMAs of the next 32 tokens are issued between the exp2 of
-// these.  Bound by MFMA and exp2 issue.  (In passes of 512 rows, each a launch that staged
-// every tile again, a 512-token chunk of 7 heads over 16 384 tokens took 8 x 17.5 us.)
+// these.  Bound by MFMA, VALU and exp2 issue, which add up.  (In passes of 512 rows, each a launch that staged
+// every tile again, a 512-token chunk of 7 heads over 16 384 tokens took 8 x 17.5 us, now 82; up to 512 rows score_kernel's
+// pipeline is the faster, 256 rows of 65 536 tokens of 8 heads 47 us to 79.)
 constexpr int MS_NT = 512, MS_WAVES = MS_NT / 64, MS_TILES = 7;
 
 template <int D>
@@ -1127,15 +1128,13 @@ __global__ void __launch_bounds__(MS_NT) mass_rows_kernel(ScoreArgs a, int items
     for (int i = lane; i < MS_TILES * TILE; i += 64) sm.sum[wave][i] = 0.f;
     __syncthreads();
 
-    // pairs p = wave / share, ... of row tiles; with fewer pairs than waves `share` waves take a
-    // pair, each every share-th 32-token unit
+    // pairs of row tiles p = wave, wave + 8, ..., each over every 32-token unit
     const int T = a.T, T2 = a.T2, R2 = a.R2, R = a.R;
     const int npair = (R2 + 63) / 64;
-    const int share = npair >= MS_WAVES ? 1 : npair >= 3 ? 2 : npair == 2 ? 4 : 8;
     const int units = 2 * nt;
     const float sl2 = a.sl2;
     float *sum = sm.sum[wave], *crow = sm.crow[wave];
-    for (int p = wave / share; p < npair; p += MS_WAVES / share) {
+    for (int p = wave; p < npair; p += MS_WAVES) {
         bf16x8_t qf[2][NKS];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
@@ -1198,18 +1197,14 @@ __global__ void __launch_bounds__(MS_NT) mass_rows_kernel(ScoreArgs a, int items
         constexpr std::true_type yes{};
         constexpr std::false_type no{};
         f32x16_t sa[2], sb[2];
-        int u = wave % share;
-        if (u < units) body(0, u, sb, sa, yes, no);
-        for (; u + 2 * share < units; u += 2 * share) {
-            body(u, u + share, sa, sb, yes, yes);
-            body(u + share, u + 2 * share, sb, sa, yes, yes);
+        int u = 0;
+        body(0, 0, sb, sa, yes, no);
+        for (; u + 2 < units; u += 2) {
+            body(u, u + 1, sa, sb, yes, yes);
+            body(u + 1, u + 2, sb, sa, yes, yes);
         }
-        if (u + share < units) {
-            body(u, u + share, sa, sb, yes, yes);
-            body(u + share, 0, sb, sa, no, yes);
-        } else if (u < units) {
-            body(u, 0, sa, sb, no, yes);
-        }
+        body(u, u + 1, sa, sb, yes, yes);   // (two units a tile)
+        body(u + 1, 0, sb, sa, no, yes);
     }
     __syncthreads();
     const float inv = 1.0f / (float)R2;

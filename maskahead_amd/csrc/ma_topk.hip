@@ -9,8 +9,12 @@
 //     the contest runs over the first m = n - W entries as a top-(C - W), and index order
 //     is position order; a row whose positions do not increase strictly gets status 1.
 //
-// A row is cut into C chunks of CS = 256 * VPT elements; workgroup (c, row) owns chunk c
-// in all three kernels, so a chunk is re-read from the L2 of the XCD that read it first.
+// A row is cut into C chunks of CS = 256 * VPT elements; workgroup (g, row) owns the run of
+// `cpw` chunks from g * cpw in all three kernels, so a chunk is re-read from the L2 of the XCD
+// that read it first.  A few rows take one chunk a workgroup: each step is then one latency.
+// Many rows (every layer's keep set at once) would run several dispatch waves of workgroups
+// that each repeat their row's decisions, so they take longer runs, the next chunk's keys
+// loaded while one is worked on: 112 rows of 32 800 keys, 3 696 chunks, HISTT.
 // Elements are monotone 32-bit keys (larger float -> larger key, -0.0 == +0.0, NaN above
 // +inf, dead slots -inf); the k-th largest key T is found digit by digit, 13 + 11 + 8 bits:
 //   1. hist:     every chunk adds its 13-bit histogram into the row's global histogram
@@ -35,6 +39,8 @@
 // Row r's histogram is block r of a state buffer that must be zero before its first use;
 // each call clears its rows' blocks again, so a state buffer of R blocks serves every
 // later call of up to R rows.  Chunk records and candidates go to a scratch workspace.
+#include <algorithm>
+
 #include "ma_common.h"
 
 namespace {
@@ -74,7 +80,7 @@ struct TopkArgs {
     int64_t rank_stride;
     const uint8_t *mask;
     int64_t mask_stride;
-    int n, k, C, vec;
+    int n, k, C, cpw, vec;
     int64_t *idx;
     int64_t idx_stride;
     float *values;
@@ -231,14 +237,21 @@ __device__ __forceinline__ void find_digit(const uint32_t (&h)[PB], uint32_t kk,
 template <int VPT, bool KEEP>
 __global__ void __launch_bounds__(TB) topk_hist_kernel(TopkArgs a) {
     __shared__ uint32_t h[H0];
-    const int c = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+    const int row = blockIdx.y, tid = threadIdx.x;
+    const int c0 = blockIdx.x * a.cpw, c1 = min(c0 + a.cpw, a.C);
     for (int i = tid; i < H0 / 4; i += TB) ((uint4 *)h)[i] = make_uint4(0u, 0u, 0u, 0u);
     uint32_t key[VPT];
-    chunk_keys<VPT, KEEP>(a, row, c, key);
+    chunk_keys<VPT, KEEP>(a, row, c0, key);
     __syncthreads();
+    for (int c = c0; c < c1; ++c) {
+        uint32_t next[VPT];
+        if (c + 1 < c1) chunk_keys<VPT, KEEP>(a, row, c + 1, next);
 #pragma unroll
-    for (int e = 0; e < VPT; ++e)
-        if (key[e]) atomicAdd(&h[key[e] >> S0], 1u);
+        for (int e = 0; e < VPT; ++e)
+            if (key[e]) atomicAdd(&h[key[e] >> S0], 1u);
+#pragma unroll
+        for (int e = 0; e < VPT; ++e) key[e] = next[e];
+    }
     __syncthreads();
     uint32_t *gh = a.state[row].hist;
     for (int i = tid; i < H0; i += TB) {
@@ -252,7 +265,8 @@ template <int VPT, bool KEEP>
 __global__ void __launch_bounds__(TB) topk_boundary_kernel(TopkArgs a) {
     constexpr int CS = TB * VPT, PB = H0 / TB;
     __shared__ uint32_t wsum[TW], found[2];
-    const int c = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+    const int row = blockIdx.y, tid = threadIdx.x;
+    const int c0 = blockIdx.x * a.cpw, c1 = min(c0 + a.cpw, a.C);
     // thread t: bins [32t, 32t + 32), loaded together with the chunk's keys
     uint32_t cnt[PB];
     const uint4 *g4 = (const uint4 *)(a.state[row].hist + tid * PB);
@@ -266,34 +280,42 @@ __global__ void __launch_bounds__(TB) topk_boundary_kernel(TopkArgs a) {
     }
     uint32_t key[VPT];
     bool bad = false;
-    chunk_keys<VPT, KEEP>(a, row, c, key, &bad);
+    chunk_keys<VPT, KEEP>(a, row, c0, key, &bad);
     find_digit<PB>(cnt, (uint32_t)a.k, wsum, found);
     const uint32_t d0 = found[0], krem = (uint32_t)a.k - found[1];
-    uint32_t packed[1] = {0u};   // low 16 bits: keys above bin d0; high: keys in bin d0
+    for (int c = c0; c < c1; ++c) {
+        uint32_t next[VPT];
+        bool next_bad = false;
+        if (c + 1 < c1) chunk_keys<VPT, KEEP>(a, row, c + 1, next, &next_bad);
+        uint32_t packed[1] = {0u};   // low 16 bits: keys above bin d0; high: keys in bin d0
 #pragma unroll
-    for (int e = 0; e < VPT; ++e) {
-        const uint32_t d = key[e] >> S0;
-        packed[0] += key[e] && d > d0 ? 1u : 0u;
-        packed[0] += key[e] && d == d0 ? 0x10000u : 0u;
-    }
-    const uint32_t total = block_prefix_runs<1>(packed, wsum);
-    uint32_t *L = a.cand + ((int64_t)row * a.C + c) * CS;
-    uint32_t pos = packed[0] >> 16;
-#pragma unroll
-    for (int e = 0; e < VPT; ++e) {
-        if (key[e] && (key[e] >> S0) == d0) {
-            L[pos] = key[e];
-            ++pos;
+        for (int e = 0; e < VPT; ++e) {
+            const uint32_t d = key[e] >> S0;
+            packed[0] += key[e] && d > d0 ? 1u : 0u;
+            packed[0] += key[e] && d == d0 ? 0x10000u : 0u;
         }
-    }
-    const bool chunk_bad = KEEP && __syncthreads_or(bad);
-    if (tid == 0) {
-        ChunkInfo ci;
-        ci.gt = (total & 0xffffu) | (chunk_bad ? 0x80000000u : 0u);
-        ci.ncand = total >> 16;
-        ci.d0 = d0;
-        ci.krem = krem;
-        a.chunk[(int64_t)row * a.C + c] = ci;
+        const uint32_t total = block_prefix_runs<1>(packed, wsum);
+        uint32_t *L = a.cand + ((int64_t)row * a.C + c) * CS;
+        uint32_t pos = packed[0] >> 16;
+#pragma unroll
+        for (int e = 0; e < VPT; ++e) {
+            if (key[e] && (key[e] >> S0) == d0) {
+                L[pos] = key[e];
+                ++pos;
+            }
+        }
+        const bool chunk_bad = KEEP && __syncthreads_or(bad);
+        if (tid == 0) {
+            ChunkInfo ci;
+            ci.gt = (total & 0xffffu) | (chunk_bad ? 0x80000000u : 0u);
+            ci.ncand = total >> 16;
+            ci.d0 = d0;
+            ci.krem = krem;
+            a.chunk[(int64_t)row * a.C + c] = ci;
+        }
+#pragma unroll
+        for (int e = 0; e < VPT; ++e) key[e] = next[e];
+        bad = next_bad;
     }
 }
 
@@ -335,7 +357,9 @@ struct EmitSmem {
     uint32_t acnt[MAX_CHUNKS];      // per chunk: candidates above T
     uint32_t ecnt[MAX_CHUNKS];      // per chunk: candidates equal to T
     uint32_t wsum[4 * TW], found[2];   // (block_prefix_runs<NR> uses NR * TW)
-    uint32_t base, take, eq;        // this workgroup's chunk
+    uint32_t take;                  // (slot-speculative path) T-equal keys the row takes
+    // (the decisions end with, per chunk: pre = output base, acnt = T-equal keys taken, ecnt =
+    // T-equal keys)
     uint32_t thr;                   // T (slot-speculative path)
     alignas(16) uint32_t hist2[H2]; // level 2 (slot-speculative path; read as uint4)
     uint32_t ncn[SPEC_C], gtc[SPEC_C];   // per chunk: candidates, keys above bin d0 (same)
@@ -351,7 +375,8 @@ __global__ void __launch_bounds__(TB) topk_emit_kernel(TopkArgs a) {
     constexpr int NR = VPT / 4, CS = TB * VPT;
     __shared__ EmitSmem S;
     __shared__ uint32_t sj[CS], sk[CS];
-    const int c = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, C = a.C;
+    const int row = blockIdx.y, tid = threadIdx.x, C = a.C;
+    const int c0 = blockIdx.x * a.cpw, c1 = min(c0 + a.cpw, C);
     const ChunkInfo *info = a.chunk + (int64_t)row * C;
     // chunk records of chunks [4t, 4t + 4) and the chunk's keys, loads in flight together
     uint32_t gt[4], nc[4];
@@ -386,12 +411,12 @@ __global__ void __launch_bounds__(TB) topk_emit_kernel(TopkArgs a) {
         spk[i] = spec_try && (e >> pl) < C ? L[(int64_t)(e >> pl) * CS + (e & (P - 1))] : 0u;
     }
     uint32_t key[VPT];
-    chunk_keys<VPT, KEEP>(a, row, c, key);
+    chunk_keys<VPT, KEEP>(a, row, c0, key);
     if constexpr (KEEP) {
         // workgroup 0 of the row: the order flag of the row and the W newest entries after
         // the selected ones
         const bool row_bad = __syncthreads_or(any_bad);
-        if (c == 0) {
+        if (c0 == 0) {
             if (tid == 0 && a.status) a.status[row] = row_bad ? 1 : 0;
             int64_t *wout = a.idx + (int64_t)row * a.idx_stride + a.k;
             for (int i = tid; i < a.w; i += TB) wout[i] = (int64_t)(a.m + i);
@@ -468,11 +493,8 @@ __global__ void __launch_bounds__(TB) topk_emit_kernel(TopkArgs a) {
             const uint32_t take = need > ebefore ? min(need - ebefore, ec) : 0u;
             const uint32_t sel = ln < C ? S.gtc[ln] + ac + take : 0u;
             const uint32_t sbefore = ma_wave_prefix_u32(sel) - sel;
-            if (ln == c) {
-                S.base = sbefore;
-                S.take = take;
-                S.eq = ec;
-            }
+            S.pre[ln] = sbefore;
+            S.acnt[ln] = take;
         }
     } else {
     uint32_t run[1] = {nc[0] + nc[1] + nc[2] + nc[3]};
@@ -608,14 +630,14 @@ __global__ void __launch_bounds__(TB) topk_emit_kernel(TopkArgs a) {
             sel[i] = ch < C ? gt[i] + S.acnt[ch] + take[i] : 0u;
             sx[0] += sel[i];
         }
-        block_prefix_runs<1>(sx, S.wsum);
+        block_prefix_runs<1>(sx, S.wsum);   // (its barriers: every read of pre and acnt is done)
         uint32_t base = sx[0];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            if (4 * tid + i == c) {
-                S.base = base;
-                S.take = take[i];
-                S.eq = e[i];
+            const int ch = 4 * tid + i;
+            if (ch < C) {
+                S.pre[ch] = base;
+                S.acnt[ch] = take[i];
             }
             base += sel[i];
         }
@@ -623,75 +645,91 @@ __global__ void __launch_bounds__(TB) topk_emit_kernel(TopkArgs a) {
     }
     // this workgroup's share of the row's histogram, cleared for the next call (the
     // boundary kernel, its only reader, has finished)
-    for (int b = c * TB + tid; b < H0; b += C * TB) a.state[row].hist[b] = 0u;
+    for (int b = blockIdx.x * TB + tid; b < H0; b += gridDim.x * TB) a.state[row].hist[b] = 0u;
     __syncthreads();
     if (spec) thr = S.thr;
-    const uint32_t cbase = S.base, ctake = S.take, ceq = S.eq;
-    uint32_t selbits = 0;
-    if (ctake == 0u || ctake >= ceq) {
-        // none or all of the chunk's keys equal to T (padding keys 0 lie below any T)
-        const bool all_eq = ctake != 0u;
+    for (int c = c0; c < c1; ++c) {
+        uint32_t next[VPT];
+        if (c + 1 < c1) chunk_keys<VPT, KEEP>(a, row, c + 1, next);
+        const uint32_t cbase = S.pre[c], ctake = S.acnt[c], ceq = S.ecnt[c];
+        uint32_t selbits = 0;
+        if (ctake == 0u || ctake >= ceq) {
+            // none or all of the chunk's keys equal to T (padding keys 0 lie below any T)
+            const bool all_eq = ctake != 0u;
 #pragma unroll
-        for (int e = 0; e < VPT; ++e) selbits |= (uint32_t)(key[e] > thr || (all_eq && key[e] == thr)) << e;
-    } else {
-        // the first `take` keys equal to T in index order
-        uint32_t eb[NR];
+            for (int e = 0; e < VPT; ++e) selbits |= (uint32_t)(key[e] > thr || (all_eq && key[e] == thr)) << e;
+        } else {
+            // the first `take` keys equal to T in index order
+            uint32_t eb[NR];
 #pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            eb[q] = 0u;
+            for (int q = 0; q < NR; ++q) {
+                eb[q] = 0u;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) eb[q] += key[4 * q + i] == thr ? 1u : 0u;
+                for (int i = 0; i < 4; ++i) eb[q] += key[4 * q + i] == thr ? 1u : 0u;
+            }
+            block_prefix_runs<NR>(eb, S.wsum);
+#pragma unroll
+            for (int q = 0; q < NR; ++q) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int e = 4 * q + i;
+                    const bool is_eq = key[e] == thr;
+                    selbits |= (uint32_t)(key[e] > thr || (is_eq && eb[q] < ctake)) << e;
+                    eb[q] += is_eq ? 1u : 0u;
+                }
+            }
         }
-        block_prefix_runs<NR>(eb, S.wsum);
+        uint32_t slot[NR];
+#pragma unroll
+        for (int q = 0; q < NR; ++q) slot[q] = __popc((selbits >> (4 * q)) & 15u);
+        const uint32_t nsel = block_prefix_runs<NR>(slot, S.wsum);
 #pragma unroll
         for (int q = 0; q < NR; ++q) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int e = 4 * q + i;
-                const bool is_eq = key[e] == thr;
-                selbits |= (uint32_t)(key[e] > thr || (is_eq && eb[q] < ctake)) << e;
-                eb[q] += is_eq ? 1u : 0u;
+                if ((selbits >> e) & 1u) {
+                    sj[slot[q]] = (uint32_t)chunk_index<VPT>(c, e);
+                    sk[slot[q]] = key[e];
+                    ++slot[q];
+                }
             }
         }
-    }
-    uint32_t slot[NR];
-#pragma unroll
-    for (int q = 0; q < NR; ++q) slot[q] = __popc((selbits >> (4 * q)) & 15u);
-    const uint32_t nsel = block_prefix_runs<NR>(slot, S.wsum);
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = 4 * q + i;
-            if ((selbits >> e) & 1u) {
-                sj[slot[q]] = (uint32_t)chunk_index<VPT>(c, e);
-                sk[slot[q]] = key[e];
-                ++slot[q];
+        __syncthreads();
+        int64_t *out = a.idx + (int64_t)row * a.idx_stride + cbase;
+        float *vout = a.values ? a.values + (int64_t)row * a.k + cbase : nullptr;
+        const float *rr = a.rank + (int64_t)row * a.rank_stride;
+        const uint8_t *mr = a.mask ? a.mask + (int64_t)row * a.mask_stride : nullptr;
+        // (cbase + nsel <= k by construction; the bound keeps inconsistent inputs from
+        // writing past the row)
+        const uint32_t nout = cbase < (uint32_t)a.k ? min(nsel, (uint32_t)a.k - cbase) : 0u;
+        for (uint32_t i = tid; i < nout; i += TB) {
+            const uint32_t j = sj[i];
+            out[i] = (int64_t)j;
+            if (vout) {
+                // the selected value from its key; a zero or NaN key re-reads the element so
+                // that -0.0 and NaN payloads come back as stored
+                float x = key_value(sk[i]);
+                if (x == 0.f || x != x) x = (mr && !mr[j]) ? -INFINITY : rr[j];
+                vout[i] = x;
             }
         }
-    }
-    __syncthreads();
-    int64_t *out = a.idx + (int64_t)row * a.idx_stride + cbase;
-    float *vout = a.values ? a.values + (int64_t)row * a.k + cbase : nullptr;
-    const float *rr = a.rank + (int64_t)row * a.rank_stride;
-    const uint8_t *mr = a.mask ? a.mask + (int64_t)row * a.mask_stride : nullptr;
-    // (cbase + nsel <= k by construction; the bound keeps inconsistent inputs from
-    // writing past the row)
-    const uint32_t nout = cbase < (uint32_t)a.k ? min(nsel, (uint32_t)a.k - cbase) : 0u;
-    for (uint32_t i = tid; i < nout; i += TB) {
-        const uint32_t j = sj[i];
-        out[i] = (int64_t)j;
-        if (vout) {
-            // the selected value from its key; a zero or NaN key re-reads the element so
-            // that -0.0 and NaN payloads come back as stored
-            float x = key_value(sk[i]);
-            if (x == 0.f || x != x) x = (mr && !mr[j]) ? -INFINITY : rr[j];
-            vout[i] = x;
-        }
+#pragma unroll
+        for (int e = 0; e < VPT; ++e) key[e] = next[e];
+        if (c + 1 < c1) __syncthreads();   // sj and sk are reused
     }
 }
 
 int topk_vpt(int n) { return n <= TB * 4 * MAX_CHUNKS ? 4 : (n <= TB * 16 * MAX_CHUNKS ? 16 : 0); }
+
+// Chunks per workgroup: one while the chip holds a workgroup for every chunk (two a CU, by the
+// emit kernel's LDS), else as many as bring the rows' workgroups down to that.
+int chunks_per_wg(int rows, int C) {
+    const int slots = 2 * ma_num_cus();
+    if ((int64_t)rows * C <= slots) return 1;
+    const int per_row = std::max(1, slots / rows);
+    return (C + per_row - 1) / per_row;
+}
 
 int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
@@ -739,6 +777,7 @@ int topk_prepare(TopkArgs &a, int &vpt, const char *who, const float *rank, int6
     a.n = n;
     a.k = k;
     a.C = (n + TB * vpt - 1) / (TB * vpt);
+    a.cpw = chunks_per_wg(rows, a.C);
     a.vec = ((uintptr_t)rank & 15) == 0 && rank_stride % 4 == 0;
     a.idx = idx;
     a.idx_stride = idx_stride;
@@ -752,7 +791,7 @@ int topk_prepare(TopkArgs &a, int &vpt, const char *who, const float *rank, int6
 // pass), so the histogram launch is skipped
 template <bool KEEP>
 int topk_launch(const TopkArgs &a, int rows, int vpt, hipStream_t st, const char *who, bool hist_ready = false) {
-    const dim3 grid(a.C, rows);
+    const dim3 grid((a.C + a.cpw - 1) / a.cpw, rows);
     if (vpt == 4) {
         if (!hist_ready) hipLaunchKernelGGL((topk_hist_kernel<4, KEEP>), grid, dim3(TB), 0, st, a);
         hipLaunchKernelGGL((topk_boundary_kernel<4, KEEP>), grid, dim3(TB), 0, st, a);
@@ -816,9 +855,10 @@ extern "C" int ma_topk_level0_into_state(const float *rank, int64_t rank_stride,
     a.mask_stride = mask_stride;
     a.n = n;
     a.C = (n + TB * vpt - 1) / (TB * vpt);
+    a.cpw = chunks_per_wg(rows, a.C);
     a.vec = ((uintptr_t)rank & 15) == 0 && rank_stride % 4 == 0;
     a.state = (RowState *)state;
-    const dim3 grid(a.C, rows);
+    const dim3 grid((a.C + a.cpw - 1) / a.cpw, rows);
     if (vpt == 4) hipLaunchKernelGGL((topk_hist_kernel<4, false>), grid, dim3(TB), 0, (hipStream_t)stream, a);
     else hipLaunchKernelGGL((topk_hist_kernel<16, false>), grid, dim3(TB), 0, (hipStream_t)stream, a);
     return ma_check_launch("ma_topk_level0_into_state");
