@@ -2,9 +2,9 @@
 // of a KV head's GQA group (the reference's splitk_attention, splitk.py:493-579).
 //
 // Pass 1 (splitk_fwd_kernel): one workgroup = one (batch, KV head) lane x one token range
-// (a prefix split, or the current block) x up to 7 row tiles of 32 query rows; 8 waves of
+// (a prefix split, or the current block) x up to 8 row tiles of 32 query rows; 8 waves of
 // up to 256 VGPRs, software-pipelined over 64-token tiles with one barrier per tile:
-//   waves 0..6   one row tile each.  S^T = K Q^T with v_mfma_f32_32x32x16_bf16 (A = K rows
+//   waves 0..7   one row tile each.  S^T = K Q^T with v_mfma_f32_32x32x16_bf16 (A = K rows
 //                from LDS, B = Q^T held in registers), so a lane owns ONE query row and 16
 //                tokens of each 32-token half; online softmax with a lazily raised
 //                reference max; O^T = alpha * O^T + V^T P^T with P^T straight from the
@@ -23,7 +23,7 @@ using namespace ma;
 
 namespace {
 
-constexpr int MAXS = 7;                     // row tiles (compute waves) per workgroup
+constexpr int MAXS = 8;                     // row tiles (compute waves) per workgroup
 // a row's running reference max is raised only when a tile's max exceeds it by more than
 // 2^8 in exp2 units, so most tiles skip the accumulator rescale; p <= 2^8 stays exact
 constexpr float LAZY_LOG2 = 8.0f;
@@ -37,6 +37,7 @@ struct FwdArgs {
     // written to slots slot0 + split; with_tail: then the workgroups of a packed prefix's
     // tail, tokens [tok_end, tail_end) to slot slot0 + nsp; with_cur: then the current block's
     int nsp, slot0, tok_beg, tok_end, with_tail, tail_end, with_cur;
+    int group_tiles;   // row tiles of a row group (the last may have fewer)
     float sl2;  // scale * log2(e)
     float scale;
     // partials of every (lane, slot, row), slot = split or nsplit (current block):
@@ -398,9 +399,9 @@ __device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, 
     const int np = cur ? 0 : L.nq - beg;                   // its packed tokens: 0 or one group
     const uint8_t *mask = cur ? nullptr : L.mask;
     const int nt = (ntok + TILE - 1) / TILE;
-    const int nS = min(MAXS, a.row_tiles - wk.rg * MAXS);
+    const int nS = min(a.group_tiles, a.row_tiles - wk.rg * a.group_tiles);
     const bool is_s = wave < nS;
-    const int rtile = wk.rg * MAXS + wave;
+    const int rtile = wk.rg * a.group_tiles + wave;
     const int row = rtile * 32 + c32;
     const bool row_ok = row < a.R;
     const int qpos = a.q_pos0 + (row_ok ? row % a.T : 0);
@@ -525,9 +526,9 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
         }
     }
 
-    const int nS = min(MAXS, a.row_tiles - wk.rg * MAXS);
+    const int nS = min(a.group_tiles, a.row_tiles - wk.rg * a.group_tiles);
     const bool is_s = wave < nS;
-    const int rtile = wk.rg * MAXS + wave;
+    const int rtile = wk.rg * a.group_tiles + wave;
     const int row = rtile * 32 + c32;
     const bool row_ok = row < a.R;
     const bool is_k = tid < KLANES;
@@ -1024,26 +1025,72 @@ Parts parts_of(int nq, int nf) {
     return p;
 }
 
-// Tokens per split: about one workgroup per CU (a workgroup's 256 VGPRs per lane and
-// 108 KB of LDS fill a CU), with
-// one CU per (lane, row group) left for the current block's workgroups, and one for a packed
-// prefix's tail, so every
-// workgroup of the launch runs in the first dispatch wave; at least one 64-token tile.
-// (Where many row groups leave few splits, a tail's CU would lengthen every split by a good
-// part; the tail then runs beside the splits of other CUs' second dispatch wave.)
-// Short prefixes (a sub-step's 2 048 selected entries) thus spread over many CUs: each
-// workgroup's cost is mostly fixed latency, so more, shorter splits finish sooner
-// (22.1 -> 17.9 us per sub-step at 4 KV heads x 2 048 entries, measured).
-int choose_split(int nq, int nf, int BH, int row_groups, int split_tokens) {
-    if (split_tokens > 0) return split_tokens;
-    const int units = BH * row_groups, n = nq + nf;
-    int per = ma_num_cus() / units - 1;
-    if (per > 8 && parts_of(nq, nf).tail()) --per;
-    if (per < 1) per = 1;
-    int sn = (n + per - 1) / per;
-    sn = ((sn + TILE - 1) / TILE) * TILE;
-    if (sn < TILE) sn = TILE;
-    return sn;
+// Where the library keeps the partials of calls without a workspace.
+constexpr int64_t NOALLOC_SCRATCH_BYTES = 32ll << 20;
+
+int64_t partial_bytes(int BH, int slots, int R, int D) {
+    const int64_t rows = (int64_t)BH * (slots + 1) * R;
+    return rows * 4 * 3 + rows * D * 2 + 256;
+}
+
+// Tokens per split and row groups.  A workgroup's 256 VGPRs per lane and 137 KB of LDS fill a
+// CU, so a launch runs in dispatch waves of one workgroup per CU.  The choice is the one whose
+// workgroups are estimated to end first: the splits', and those of the current block and of a
+// packed prefix's tail, which run on CUs the splits leave free.  Counted in token tiles: a
+// split costs its tiles and about 3 more (its first loads, its partial), a short segment 6 and,
+// where it is not pipelined, twice its tiles; and counted on one XCD, since the workgroups go
+// to the XCDs in turn and wait there even if another has a free CU.  Candidates: row groups of
+// at most 7 row tiles, or of 8, whose tiles take 1.15 times as long (the eighth wave only
+// stages otherwise); as many splits as one dispatch wave holds, with or without the other
+// workgroups.  (Two waves of half the splits cost their first loads twice: 9 000 x 64, 84 row
+// tiles, 218 us for 182.)  The first, 7 row tiles with everything in the wave, stays unless
+// another is estimated to be faster by a twentieth.  A prefill chunk of 512 tokens, two layers,
+// before (7 row tiles, room for one short segment a row group) and now: 28 heads of 128 over 4
+// x 16 384 packed 528 -> 460 us (14 groups in 4 splits for 16 in 3), 32 heads over 8 x 14 000
+// 612 -> 541, 32 heads of 64 over 8 x 10 000 packed 342 -> 279.  Short prefixes (a sub-step's
+// 2 048 selected entries) spread over many CUs: each workgroup's cost is mostly fixed latency,
+// so more, shorter splits finish sooner (22.1 -> 17.9 us per sub-step at 4 KV heads x 2 048).
+constexpr int XCDS = 8;
+
+struct Split {
+    int tokens, groups;   // a multiple of 64, and row groups, of equal size as far as whole tiles allow
+};
+
+Split choose_split(int nq, int nf, int BH, int row_tiles, int T, int R, int D, int split_tokens) {
+    const int groups7 = (row_tiles + 6) / 7;
+    if (split_tokens > 0) return {split_tokens, groups7};
+    const int cus = ma_num_cus(), n = nq + nf, nt = max(1, (n + TILE - 1) / TILE);
+    const bool tail = parts_of(nq, nf).tail();
+    const int64_t cu = max(1, cus / XCDS);   // of one XCD
+    const int64_t tcur = 6 + (T + TILE - 1) / TILE * (nq ? 2 : 1), ttail = tail ? 6 + 2 : 0;
+    auto span = [&](int groups, int s) {
+        const int64_t units = (int64_t)BH * groups, other = (units + XCDS - 1) / XCDS;
+        const int64_t w = (units * s + XCDS - 1) / XCDS, t = 3 + (nt + s - 1) / s, waves = (w + cu - 1) / cu;
+        const int64_t room = (cu - 1 - (w - 1) % cu) * t, work = other * (tcur + ttail);
+        const int64_t late = work > room ? max(tcur, (work - room + cu - 1) / cu) : 0;
+        return max(waves * t + late, (waves - 1) * t + tcur) * ((row_tiles + groups - 1) / groups > 7 ? 115 : 100);
+    };
+    // more splits than one wave of 7-tile workgroups has are taken only while the partials fit
+    // the array kept for calls without a workspace, so that no call outgrows it by this choice
+    const int few = max(1, cus / (BH * groups7) - 1);
+    Split best{0, 0};
+    int64_t best_span = 0;
+    for (int tiles = 7; tiles <= MAXS; ++tiles) {
+        const int groups = (row_tiles + tiles - 1) / tiles, units = BH * groups;
+        if (tiles > 7 && groups == groups7) break;
+        for (int with = 1; with >= 0; --with) {
+            int s = max(1, min((cus - with * units * (tail ? 2 : 1)) / units, nt));
+            // slots: the splits (packed and 16-bit ones both rounded up) and a tail
+            if (s > few && partial_bytes(BH, s + 2, R, D) > NOALLOC_SCRATCH_BYTES) s = min(few, nt);
+            const int per = (nt + s - 1) / s;
+            const int64_t sp = span(groups, (nt + per - 1) / per);
+            if (best.groups == 0 || 20 * sp < 19 * best_span) {
+                best = {per * TILE, groups};
+                best_span = sp;
+            }
+        }
+    }
+    return best;
 }
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
@@ -1058,19 +1105,12 @@ static int slot_count(int nq, int nf, int sn) {
     return p.splits(sn) + (p.tail() ? 1 : 0) + p.fsplits(nq, nf, sn);
 }
 
-static int row_groups_of(int Hq, int H, int T) {
-    const int row_tiles = ((Hq / H) * T + 31) / 32;
-    return (row_tiles + MAXS - 1) / MAXS;
-}
-
 extern "C" int64_t ma_splitk_workspace_bytes(int B, int H, int Hq, int T, int D, int nq, int nf,
                                              int split_tokens) {
     if (B <= 0 || H <= 0 || Hq <= 0 || Hq % H || T <= 0 || D <= 0 || nq < 0 || nf < 0) return -1;
     const int R = (Hq / H) * T;
-    const int sn = choose_split(nq, nf, B * H, row_groups_of(Hq, H, T), split_tokens);
-    const int nsplit = slot_count(nq, nf, sn);
-    const int64_t rows = (int64_t)B * H * (nsplit + 1) * R;
-    return rows * 4 * 3 + rows * D * 2 + 256;
+    const int sn = choose_split(nq, nf, B * H, (R + 31) / 32, T, R, D, split_tokens).tokens;
+    return partial_bytes(B * H, slot_count(nq, nf, sn), R, D);
 }
 
 namespace {
@@ -1112,8 +1152,8 @@ int make_plan(Plan &pl, const char *who, ma_tensor4 q, int B, int Hq, int T, int
     const int G = Hq / H;
     const int R = G * T;
     const int row_tiles = (R + 31) / 32;
-    const int row_groups = (row_tiles + MAXS - 1) / MAXS;
-    const int sn = choose_split(p->nq, p->nf, B * H, row_groups, split_tokens);
+    const Split split = choose_split(p->nq, p->nf, B * H, row_tiles, T, R, D, split_tokens);
+    const int row_groups = split.groups, sn = split.tokens;
     const int nsplit = slot_count(p->nq, p->nf, sn);
     const int64_t need = ma_splitk_workspace_bytes(B, H, Hq, T, D, p->nq, p->nf, sn);
     if (workspace_bytes < need) {
@@ -1142,6 +1182,7 @@ int make_plan(Plan &pl, const char *who, ma_tensor4 q, int B, int Hq, int T, int
     fa.c_pos0 = c_pos0;
     fa.row_tiles = row_tiles;
     fa.row_groups = row_groups;
+    fa.group_tiles = (row_tiles + row_groups - 1) / row_groups;   // as equal as whole tiles allow
     fa.BH = B * H;
     fa.scale = scale;
     fa.sl2 = scale * MA_LOG2E;
@@ -1183,12 +1224,13 @@ int launch_partial_d(const Plan &pl, hipStream_t st) {
         fa.tok_end = nq + nf;
         fa.with_tail = 0;
         fa.with_cur = 1;
+        const dim3 grid((nsf + 1) * units);
         const bool bf = (nf == 0 || fa.pre.fdtype == MA_BF16) &&
                         (fa.Tc == 0 || (fa.kc.dtype == MA_BF16 && fa.vc.dtype == MA_BF16));
         if (bf)
-            hipLaunchKernelGGL((splitk_fwd_kernel<D, 2, true>), dim3((nsf + 1) * units), dim3(NTH), 0, st, fa);
+            hipLaunchKernelGGL((splitk_fwd_kernel<D, 2, true>), grid, dim3(NTH), 0, st, fa);
         else
-            hipLaunchKernelGGL((splitk_fwd_kernel<D, 1, true>), dim3((nsf + 1) * units), dim3(NTH), 0, st, fa);
+            hipLaunchKernelGGL((splitk_fwd_kernel<D, 1, true>), grid, dim3(NTH), 0, st, fa);
     }
     return ma_check_launch("ma_splitk_partial");
 }
@@ -1275,7 +1317,6 @@ extern "C" int ma_splitk_attention(ma_tensor4 q, int B, int Hq, int T, int D, co
 // merge reads.  Calls that overlap in time on one device share the array and race.
 namespace {
 
-constexpr int64_t NOALLOC_SCRATCH_BYTES = 32ll << 20;
 __device__ __align__(256) uint8_t scratch[NOALLOC_SCRATCH_BYTES];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
