@@ -145,7 +145,7 @@ int ma_value_centre(const void *op, int op_dtype, int B, int H, int G, int T, in
  * v_round: 0, or MA_BF16 / MA_F16: the distance reads packed V rounded to that dtype (the
  * reference reads the prefix it unpacked to the query dtype when it has one,
  * splitk.py:513-516, 592).  mass/score [B,H,n] contiguous.  Mass-only calls take any number
- * of selection rows (run in passes of at most 512, each adding its share of the mean);
+ * of selection rows (more than 512 in a kernel of their own);
  * value-aware calls take at most 512 selection rows and 1 024 rows per KV head. */
 int ma_prefix_scores(ma_tensor4 q, int B, int Hq, int T, int D, const ma_prefix *p, int H,
                      const int32_t *q_rows, int T2, const float *mp, const float *lp, const void *op,
