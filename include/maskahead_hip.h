@@ -118,10 +118,11 @@ int ma_splitk_attention(ma_tensor4 q, int B, int Hq, int T, int D, const ma_pref
 /* No counterpart in the reference: ma_splitk_attention for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments and results as ma_splitk_attention, without the workspace: the split
- * partials live in a fixed library-owned device array of ma_splitk_noalloc_max_bytes()
- * bytes (32 MiB) per device, held until the process ends.  A call whose
- * ma_splitk_workspace_bytes() exceeds it returns MA_EWORKSPACE.  The call allocates
- * nothing; the first call on a device looks up that device's copy of the array.  All calls
+ * partials live in a fixed library-owned device array (48 MiB per device, held until the
+ * process ends).  A call whose ma_splitk_workspace_bytes() exceeds
+ * ma_splitk_noalloc_max_bytes() (32 MiB) returns MA_EWORKSPACE, unless it does so only by the
+ * partial of what a packed prefix leaves behind its whole 64-token tiles, which the array
+ * holds besides.  The call allocates nothing; the first call on a device looks up that device's copy of the array.  All calls
  * on one device share the array, so calls that overlap in time on one device (two streams,
  * two host threads) race; order them on one stream. */
 int64_t ma_splitk_noalloc_max_bytes(void);

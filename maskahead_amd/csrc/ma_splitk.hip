@@ -1025,8 +1025,12 @@ Parts parts_of(int nq, int nf) {
     return p;
 }
 
-// Where the library keeps the partials of calls without a workspace.
-constexpr int64_t NOALLOC_SCRATCH_BYTES = 32ll << 20;
+// Calls without a workspace: the bytes of partials they may need, a packed prefix's tail behind
+// splits not counted, and the array that holds them.  The tail's slot is one beside at least
+// two, so half as much again holds every call within the limit; counted, it refused calls of
+// few splits and many rows (16 lanes of 3 584 rows over 65 632 packed tokens: 30.7 MB without
+// it, 46.1 with).
+constexpr int64_t NOALLOC_MAX_BYTES = 32ll << 20, NOALLOC_SCRATCH_BYTES = NOALLOC_MAX_BYTES / 2 * 3;
 
 int64_t partial_bytes(int BH, int slots, int R, int D) {
     const int64_t rows = (int64_t)BH * (slots + 1) * R;
@@ -1071,7 +1075,7 @@ Split choose_split(int nq, int nf, int BH, int row_tiles, int T, int R, int D, i
         return max(waves * t + late, (waves - 1) * t + tcur) * ((row_tiles + groups - 1) / groups > 7 ? 115 : 100);
     };
     // more splits than one wave of 7-tile workgroups has are taken only while the partials fit
-    // the array kept for calls without a workspace, so that no call outgrows it by this choice
+    // what calls without a workspace may need, so that no call outgrows it by this choice
     const int few = max(1, cus / (BH * groups7) - 1);
     Split best{0, 0};
     int64_t best_span = 0;
@@ -1081,7 +1085,7 @@ Split choose_split(int nq, int nf, int BH, int row_tiles, int T, int R, int D, i
         for (int with = 1; with >= 0; --with) {
             int s = max(1, min((cus - with * units * (tail ? 2 : 1)) / units, nt));
             // slots: the splits (packed and 16-bit ones both rounded up) and a tail
-            if (s > few && partial_bytes(BH, s + 2, R, D) > NOALLOC_SCRATCH_BYTES) s = min(few, nt);
+            if (s > few && partial_bytes(BH, s + 2, R, D) > NOALLOC_MAX_BYTES) s = min(few, nt);
             const int per = (nt + s - 1) / s;
             const int64_t sp = span(groups, (nt + per - 1) / per);
             if (best.groups == 0 || 20 * sp < 19 * best_span) {
@@ -1348,7 +1352,7 @@ int scratch_address(void **out, const char *who) {
 
 }  // namespace
 
-extern "C" int64_t ma_splitk_noalloc_max_bytes(void) { return NOALLOC_SCRATCH_BYTES; }
+extern "C" int64_t ma_splitk_noalloc_max_bytes(void) { return NOALLOC_MAX_BYTES; }
 
 extern "C" int ma_splitk_attention_noalloc(ma_tensor4 q, int B, int Hq, int T, int D, const ma_prefix *p, int H,
                                            ma_tensor4 kc, ma_tensor4 vc, int Tc, int causal_block, int q_pos0,
@@ -1360,10 +1364,14 @@ extern "C" int ma_splitk_attention_noalloc(ma_tensor4 q, int B, int Hq, int T, i
         ma_set_error("%s: bad geometry (B=%d H=%d Hq=%d T=%d D=%d)", who, B, H, Hq, T, D);
         return MA_EINVAL;
     }
-    if (need > NOALLOC_SCRATCH_BYTES) {
-        ma_set_error("%s: this call needs %lld bytes of split partials, above the library's fixed %lld-byte "
+    const Parts pt = parts_of(p->nq, p->nf);
+    const int R = (Hq / H) * T;
+    const int64_t slot = partial_bytes(B * H, 1, R, D) - partial_bytes(B * H, 0, R, D);
+    const int64_t tail = pt.tail() && pt.nq64 > 0 ? slot : 0;
+    if (need - tail > NOALLOC_MAX_BYTES) {
+        ma_set_error("%s: this call needs %lld bytes of split partials, above the %lld of the library's fixed "
                      "scratch; use ma_splitk_attention with a workspace",
-                     who, (long long)need, (long long)NOALLOC_SCRATCH_BYTES);
+                     who, (long long)(need - tail), (long long)NOALLOC_MAX_BYTES);
         return MA_EWORKSPACE;
     }
     void *ws = nullptr;
