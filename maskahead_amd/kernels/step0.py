@@ -103,12 +103,17 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
         raise ValueError("q_rows cannot be empty")
     dev = query.device
     stored = nat = prefix.native()
-    used, vround, copy = prefix, 0, None
+    used, vround, copy, spare = prefix, 0, None, None
     if _unpacked(prefix, r, query):
         if query.dtype == torch.float16:
             for x in (out_key, out_value):
                 if x is not None and tuple(x.shape) != (b, hkv, k, d):
                     raise ValueError("output buffer has the wrong shape")
+            # one of the two alone may be asked for: the other is gathered beside it
+            given = out_key if out_key is not None else out_value
+            if given is not None and (out_key is None or out_value is None):
+                spare = torch.empty((b, hkv, k, d), dtype=given.dtype, device=dev)
+                out_key, out_value = (spare, out_value) if out_key is None else (out_key, spare)
             # the f16 copy the reference reads (K and V rounded f32 -> f16, then f16 -> bf16 at
             # every dot), made in the workspace owner's storage: as splitk_attention's, without
             # an allocation and a Python call per stage (93 -> 70 us a layer at 8 192 tokens)
@@ -145,6 +150,6 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
     result = (out, (mp, lp, op, used), mass, score, idx)
     # the plan keeps every tensor its pointers name alive: q_rows (a cached device table, or
     # None), the select state, the workspace and the f16 copy (which another layer sharing
-    # the owner may have replaced by larger ones since)
-    bufs._plan = (prefix, workspace, key, rows_key, args, result, stored, copy, q_rows, st, ws)
+    # the owner may have replaced by larger ones since), and the output nobody asked for
+    bufs._plan = (prefix, workspace, key, rows_key, args, result, stored, copy, q_rows, st, ws, spare)
     return result

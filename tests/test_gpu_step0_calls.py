@@ -1,10 +1,10 @@
-"""What one-call step 0 checks: output buffers of the wrong shape (f16 queries over a packed
-prefix, which read an f16 copy)."""
+"""What one-call step 0 checks and takes: output buffers of the wrong shape and a single output
+(f16 queries over a packed prefix, which read an f16 copy)."""
 
 import pytest
 import torch
 
-from maskahead_amd.kernels import Step0Buffers, step0_select
+from maskahead_amd.kernels import Step0Buffers, gather_packed_kv, step0_select
 
 from _util import gpu_prefix, layer_inputs, packed_cpu
 
@@ -32,3 +32,14 @@ def test_output_of_the_wrong_shape(gpu):
         for kw in (dict(out_key=bad, out_value=good), dict(out_key=good, out_value=bad), dict(out_key=bad)):
             with pytest.raises(ValueError):
                 _step0(Step0Buffers(), layer, **kw)
+
+
+@pytest.mark.parametrize("name", ["out_key", "out_value"])
+def test_one_output_alone(gpu, name):
+    layer = _layer(gpu, 2)
+    bufs = Step0Buffers()
+    for dtype in (torch.float16, torch.float16, torch.bfloat16):     # the second call repeats the first
+        got = torch.full((1, 2, K, D), float("nan"), dtype=dtype, device=gpu)
+        _, stats, _, _, idx = _step0(bufs, layer, **{name: got})
+        both = gather_packed_kv(stats[3], idx, dtype=dtype)
+        assert torch.equal(got, both[name == "out_value"])
