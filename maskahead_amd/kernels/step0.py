@@ -13,13 +13,21 @@ import torch
 
 from .. import _native as N
 from .select import _state
-from .splitk import Prefix
+from .splitk import Prefix, dequantize_prefix
 
 
 def _unpacked(prefix: Prefix, r: int, query: torch.Tensor) -> bool:
     """Whether the reference reads this packed prefix through a copy unpacked to the
     query dtype (splitk.py:513-516), as splitk_attention does."""
     return bool(prefix.nq) and (r > 256 or prefix.n > 256) and query.dtype != torch.float32
+
+
+def _f16_copy(prefix: Prefix, query: torch.Tensor, current_key: torch.Tensor) -> Prefix:
+    """The f16 copy of a packed prefix that the reference reads for f16 queries (K and V
+    rounded f32 -> f16, then f16 -> bf16 at every dot), as splitk_attention makes it: a
+    statistics tuple names it, so every call has its own."""
+    kv = dequantize_prefix(prefix, query.shape[0], current_key.shape[1], query.shape[3], dtype=torch.float16)
+    return Prefix.dense(*kv, mask=prefix.mask)
 
 
 class Step0Buffers:
@@ -52,9 +60,9 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
     call.  rows: the selection rows (a host list -- 0 .. T2-1 in order needs no table --
     or an int32 device tensor).  out_key / out_value (optional): [B, Hkv, k, D] views the
     selected entries are gathered into (the layer's compact buffer).  workspace: where the
-    scratch workspace lives (default bufs), the f16 copy of a packed prefix among it
-    (prefix_used names that copy: valid until the owner's next call); layers run one after
-    another on a stream can share one."""
+    scratch workspace lives (default bufs); layers run one after another on a stream can
+    share one.  An f16 query's packed prefix is read through an f16 copy: prefix_used is that
+    copy, made by this call and nobody else's."""
     stream = N.stream_of(query)
     rows_key = rows if isinstance(rows, torch.Tensor) else tuple(rows)
     views = tuple(None if x is None else (x.data_ptr(), x.shape, x.stride(), x.dtype) for x in (out_key, out_value))
@@ -66,13 +74,15 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
     if (plan is not None and plan[0] is prefix and plan[1] is workspace and plan[2] == key
             and (plan[3] is rows_key if isinstance(rows_key, torch.Tensor) else plan[3] == rows_key)
             and plan[6] is prefix.native()):
-        args, result, copy = plan[4], plan[5], plan[7]
+        args, result, copied = plan[4], plan[5], plan[7]
         # the same shapes, strides and dtypes (the key): only the operands' addresses change
         args[0].ptr = query.data_ptr()
         if current_key.shape[2]:
             args[7].ptr, args[8].ptr = current_key.data_ptr(), current_value.data_ptr()
-        if copy is not None:
-            N.check(N.load().ma_dequant_prefix(*copy), "ma_dequant_prefix")
+        if copied:
+            used = _f16_copy(prefix, query, current_key)
+            args[5].kf, args[5].vf = used.kf.data_ptr(), used.vf.data_ptr()
+            result = (result[0], (*result[1][:3], used), *result[2:])
         N.check(N.load().ma_step0(*args), "ma_step0")
         return result
     if query.ndim != 4 or current_key.ndim != 4:
@@ -103,7 +113,7 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
         raise ValueError("q_rows cannot be empty")
     dev = query.device
     stored = nat = prefix.native()
-    used, vround, copy, spare = prefix, 0, None, None
+    used, vround, copied, spare = prefix, 0, False, None
     if _unpacked(prefix, r, query):
         if query.dtype == torch.float16:
             for x in (out_key, out_value):
@@ -114,14 +124,10 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
             if given is not None and (out_key is None or out_value is None):
                 spare = torch.empty((b, hkv, k, d), dtype=given.dtype, device=dev)
                 out_key, out_value = (spare, out_value) if out_key is None else (out_key, spare)
-            # the f16 copy the reference reads (K and V rounded f32 -> f16, then f16 -> bf16 at
-            # every dot), made in the workspace owner's storage: as splitk_attention's, without
-            # an allocation and a Python call per stage (93 -> 70 us a layer at 8 192 tokens)
-            own = workspace or bufs
-            k16, v16 = (own.take(x, b * hkv * n * d, torch.float16, dev, (b, hkv, n, d)) for x in ("k16", "v16"))
-            used = Prefix.dense(k16, v16, mask=prefix.mask)
-            copy = (stored, b, hkv, d, N.t4(k16), N.t4(v16), stream)
-            nat = used.native()
+            # (a descriptor of the plan's own, which a repeated call points at its own copy: the
+            # caller may keep `used`)
+            used, copied = _f16_copy(prefix, query, current_key), True
+            nat = used._build_native()
         else:
             vround = N.dtype_code(query.dtype)
             used = prefix.with_vround(vround)
@@ -144,12 +150,11 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
             N.ptr(q_rows), t2, 1 if value else 0, 2 if value else 1, vround, mass.data_ptr(), N.ptr(score), k,
             idx.data_ptr(), N.t4(out_key), N.t4(out_value), st.data_ptr(), st.numel(), ws.data_ptr(), ws_bytes,
             stream]
-    if copy is not None:
-        N.check(N.load().ma_dequant_prefix(*copy), "ma_dequant_prefix")
     N.check(N.load().ma_step0(*args), "ma_step0")
     result = (out, (mp, lp, op, used), mass, score, idx)
     # the plan keeps every tensor its pointers name alive: q_rows (a cached device table, or
-    # None), the select state, the workspace and the f16 copy (which another layer sharing
-    # the owner may have replaced by larger ones since), and the output nobody asked for
-    bufs._plan = (prefix, workspace, key, rows_key, args, result, stored, copy, q_rows, st, ws, spare)
+    # None), the select state, the workspace (which another layer sharing the owner may have
+    # replaced by a larger one since), the output nobody asked for; not the f16 copy
+    kept = (out, (mp, lp, op, None if copied else used), mass, score, idx)
+    bufs._plan = (prefix, workspace, key, rows_key, args, kept, stored, copied, q_rows, st, ws, spare)
     return result

@@ -1,10 +1,11 @@
-"""What one-call step 0 checks and takes: output buffers of the wrong shape and a single output
-(f16 queries over a packed prefix, which read an f16 copy)."""
+"""What one-call step 0 keeps and checks between calls: output buffers of the wrong shape and
+a single output (f16 queries over a packed prefix, which read an f16 copy), and the copy that
+the statistics name."""
 
 import pytest
 import torch
 
-from maskahead_amd.kernels import Step0Buffers, gather_packed_kv, step0_select
+from maskahead_amd.kernels import Step0Buffers, gather_packed_kv, prefix_scores, splitk_attention, step0_select
 
 from _util import gpu_prefix, layer_inputs, packed_cpu
 
@@ -43,3 +44,23 @@ def test_one_output_alone(gpu, name):
         _, stats, _, _, idx = _step0(bufs, layer, **{name: got})
         both = gather_packed_kv(stats[3], idx, dtype=dtype)
         assert torch.equal(got, both[name == "out_value"])
+
+
+def test_statistics_keep_their_copy(gpu):
+    """Scores taken from one call's statistics after another layer's call, and after the same
+    layer's, over one shared workspace."""
+    ws = Step0Buffers()
+    layers = [_layer(gpu, s) for s in (3, 4)]
+    bufs = [Step0Buffers(), Step0Buffers()]
+    for call in range(2):                                            # planned, then repeated
+        kept = []
+        for b, layer in zip(bufs, layers):
+            _, stats, mass, score, _ = _step0(b, layer, workspace=ws)
+            kept.append((layer, stats[3], stats[3].kf.clone(), tuple(x.clone() for x in stats[:3]), mass.clone(), score.clone()))
+        again = _step0(bufs[0], layers[0], workspace=ws)
+        for layer, used, key, (mp, lp, op), mass, score in kept:
+            assert again[1][3] is not used and torch.equal(used.kf, key)
+            m, s = prefix_scores(layer[0], layer[3], (mp, lp, op, used), list(range(T)), value=True)
+            assert torch.equal(m, mass) and torch.equal(s, score)
+            want = splitk_attention(*layer[:1], layer[3], *layer[1:3], want_prefix=True)[1]
+            assert torch.equal(want[3].kf, used.kf) and torch.equal(want[3].vf, used.vf)
