@@ -64,15 +64,19 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
     share one.  An f16 query's packed prefix is read through an f16 copy: prefix_used is that
     copy, made by this call and nobody else's."""
     stream = N.stream_of(query)
-    rows_key = rows if isinstance(rows, torch.Tensor) else tuple(rows)
+    # rows on the device are named by the tensor, host ones by their values
+    on_device = isinstance(rows, torch.Tensor) and rows.is_cuda
+    rows_key = rows if on_device else tuple(rows.tolist() if isinstance(rows, torch.Tensor) else rows)
     views = tuple(None if x is None else (x.data_ptr(), x.shape, x.stride(), x.dtype) for x in (out_key, out_value))
     key = (query.shape, query.stride(), query.dtype, current_key.shape, current_key.stride(), current_value.stride(),
-           current_key.dtype, current_value.dtype, int(k), bool(value), scaling, views, stream)
+           current_key.dtype, current_value.dtype, int(k), bool(value), scaling, views, stream,
+           (rows.data_ptr(), rows.shape) if on_device else None)
     plan = bufs._plan
     # (prefix.native() returns the same descriptor object while the prefix's tensors and
-    # mask are the ones it was built from)
+    # mask are the ones it was built from; rows on the device are read by the kernels where the
+    # plan's table is that tensor itself, not an int32 copy of what it held then)
     if (plan is not None and plan[0] is prefix and plan[1] is workspace and plan[2] == key
-            and (plan[3] is rows_key if isinstance(rows_key, torch.Tensor) else plan[3] == rows_key)
+            and (plan[8] is rows if on_device else type(plan[3]) is tuple and plan[3] == rows_key)
             and plan[6] is prefix.native()):
         args, result, copied = plan[4], plan[5], plan[7]
         # the same shapes, strides and dtypes (the key): only the operands' addresses change
@@ -98,11 +102,11 @@ def step0_select(bufs: Step0Buffers, query: torch.Tensor, prefix: Prefix, curren
     if n <= 0 or not 0 < k <= n:
         raise ValueError(f"read budget k={k} outside [1, {n}]")
     prefix.check_mask(b, hkv)
-    if isinstance(rows, torch.Tensor) and rows.is_cuda:
+    if on_device:
         q_rows = rows.to(torch.int32).contiguous()
         t2 = int(q_rows.numel())
     else:
-        host = tuple(int(x) for x in (rows.tolist() if isinstance(rows, torch.Tensor) else rows))
+        host = tuple(int(x) for x in rows_key)
         if any(x < 0 or x >= t for x in host):
             raise ValueError(f"q_rows must be block positions in [0, {t})")
         from .splitk import _row_table

@@ -1,6 +1,6 @@
 """What one-call step 0 keeps and checks between calls: output buffers of the wrong shape and
-a single output (f16 queries over a packed prefix, which read an f16 copy), and the copy that
-the statistics name."""
+a single output (f16 queries over a packed prefix, which read an f16 copy), the copy that the
+statistics name, and selection rows changed in place."""
 
 import pytest
 import torch
@@ -64,3 +64,17 @@ def test_statistics_keep_their_copy(gpu):
             assert torch.equal(m, mass) and torch.equal(s, score)
             want = splitk_attention(*layer[:1], layer[3], *layer[1:3], want_prefix=True)[1]
             assert torch.equal(want[3].kf, used.kf) and torch.equal(want[3].vf, used.vf)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [torch.tensor([3, 7], dtype=torch.int64), torch.tensor([3, 7], dtype=torch.int32)])
+@pytest.mark.parametrize("where", ["cpu", "gpu"])
+def test_rows_changed_in_place(gpu, dtype, rows, where):
+    layer = _layer(gpu, 5, dtype)
+    rows = rows.clone() if where == "cpu" else rows.to(gpu)
+    bufs = Step0Buffers()
+    for values in ((3, 7), (3, 7), (0, 15), (2, 2)):
+        rows.copy_(torch.tensor(values))
+        got = _step0(bufs, layer, rows)
+        want = _step0(Step0Buffers(), layer, list(values))
+        assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3]) and torch.equal(got[4], want[4])
