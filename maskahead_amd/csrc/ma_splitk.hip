@@ -478,6 +478,17 @@ __device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, 
                          &S.u.o[wave][0]);
 }
 
+// The kernel's arguments, loaded where they are asked for: behind an address the compiler cannot
+// follow back.  A short segment's loads, hoisted to the top of the kernel with all others, kept
+// two lane descriptors and the whole argument struct in scalar registers at once (94 to 113 of
+// them spilled to vector lanes in the D 128 kernels, 121 and 104 at D 64; none so).
+__device__ __forceinline__ const FwdArgs &args_again() {
+    typedef __attribute__((address_space(4))) const FwdArgs *kernarg;
+    uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();   // (the first parameter)
+    asm volatile("" : "+s"(p));
+    return *(const FwdArgs *)(kernarg)p;
+}
+
 // MASK: the prefix has a slot mask (packed sources: their splits are whole 64-token tiles
 // either way, what is left goes to short_segment, so no tile needs bounds)
 template <int D, int SRC, bool MASK>
@@ -492,13 +503,14 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, c32 = lane & 31, hf = lane >> 5;
 
-    const Lane L = make_lane(a.pre, b, h, bh);
     if constexpr (SRC == 0) {
         if (wk.seg != SEG_SPLIT) {
-            short_segment<D>(a, wk, L, S);
+            const FwdArgs &args = args_again();
+            short_segment<D>(args, wk, make_lane(args.pre, b, h, bh), S);
             return;
         }
     }
+    const Lane L = make_lane(a.pre, b, h, bh);
     int n_beg, n_end;
     if (wk.cur) {
         n_beg = 0;
