@@ -202,6 +202,10 @@ struct FwdSmem {
 // tile the last of them came ~2 000 cycles after the tile itself (8 000): a sub-step over
 // 2 048 entries 16.4 -> 15.9 us.  A packed tile is a third of that and its dequantization
 // covers the wait: there the turn through LDS only cost (544 tokens 40.9 -> 41.5 us a step).
+// So it does for few row tiles, whose fragments' loads are few: sub-steps over 2 048 entries, 28
+// query heads over 4, direct and turned: 2 row tiles 11.11 and 11.44 us, 4 12.63 and 12.68, 5
+// 14.41 and 14.39, 7 15.76 and 15.25.
+constexpr int FEW_TILES = 4;
 template <int D>
 struct QRows {
     static constexpr int CH = D / 8, NI = 32 * CH / 64;
@@ -728,7 +732,7 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
     // prologue: tiles 0 and 1 staged, tile 2's loads in flight; Q of the row tile
     if (nt > 0) load_tile(0);
     bf16x8_t qf[NKS];
-    if constexpr (SRC == 0) {
+    if (SRC == 0 || nS <= FEW_TILES) {
         if (is_s) {
             const int g = row_ok ? row / a.T : 0, t = row_ok ? row % a.T : 0;
             const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
