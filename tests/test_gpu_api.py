@@ -155,7 +155,7 @@ def test_mask_of_the_wrong_shape_is_rejected(gpu):
 def test_probe_of_four_blocks_and_long_prefill_chunk(gpu):
     """A lookahead probe of 4 masked blocks (t = 128: 7 x 96 = 672 selection rows per KV
     head) and a 512-token prefill chunk with its mass (7 x 512 = 3 584 rows per KV head):
-    the mass runs in passes of at most 512 rows."""
+    the mass of more than 512 rows has a kernel of its own."""
     n, d, blk = 1024, 128, 32
     q, k, v, kc, vc = layer_inputs(b=1, hq=28, hkv=4, d=d, n=n, t=512, seed=57, dtype=torch.bfloat16)
     c, views = _cache(gpu, k, v, QuantizationConfig())

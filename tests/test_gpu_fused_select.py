@@ -3,9 +3,9 @@
 exactly what prefix_scores followed by topk_ascending returns (session.py:1418-1438):
 identical mass and score bits and identical indices, for packed and 16-bit prefixes,
 masked and unmasked, mass and score ranks, the GQA-reduced VALU pass (whose histogram
-comes from the select's own level-0 launch), mass passes over more rows than one launch
-takes, and workgroups that count their keys in several blocks.  Each call must leave the
-shared select state zero."""
+comes from the select's own level-0 launch), the mass of more rows than that pass holds (a
+kernel of its own, likewise), the instantiations of more than 8 row tiles, and workgroups
+that count their keys in several blocks.  Each call must leave the shared select state zero."""
 
 import pytest
 import torch
@@ -71,9 +71,25 @@ def test_fused_small_row_pass(gpu):
     _compare(gpu, q, p, kc, vc, [31], 512, value=True, rank="score")
 
 
+@pytest.mark.parametrize("kind", ["packed", "dense", "masked"])
+@pytest.mark.parametrize("rank", ["score", "mass"])
+def test_fused_many_row_tiles(gpu, kind, rank):
+    """448 selection rows (64 positions x G 7): 14 row tiles, the histogram built in the score
+    pass by whole tiles, the tile of an odd key group and a residual, and a ragged last one."""
+    n, nq = 2048 + 32 + 40, 2048 + 32
+    q, k, v, kc, vc = layer_inputs(hq=28, hkv=4, d=128, n=n, t=64, seed=26, dtype=torch.bfloat16)
+    mask = (torch.rand((1, 4, n), generator=torch.Generator().manual_seed(5)) >= 0.2).to(torch.uint8)
+    if kind == "dense":
+        p = Prefix.dense(k.to(gpu), v.to(gpu))
+    else:
+        store, nq = packed_cpu(k[:, :, :nq], v[:, :, :nq], pad_groups=1)
+        p = gpu_prefix(store, nq, gpu, kf=k[:, :, nq:], vf=v[:, :, nq:], mask=mask if kind == "masked" else None)
+    _compare(gpu, q, p, kc, vc, list(range(64)), 300, value=rank == "score", rank=rank)
+
+
 def test_fused_mass_passes(gpu):
-    """672 selection rows (96 positions x G 7): mass-only passes of at most 512 rows, the
-    histogram from the last pass's final mass."""
+    """672 selection rows (96 positions x G 7): more than the score pass holds, so the mass has a
+    kernel of its own and the histogram is the select's own launch over it."""
     q, k, v, kc, vc = layer_inputs(hq=28, hkv=4, d=128, n=4096, t=96, seed=24, dtype=torch.bfloat16)
     store, nq = packed_cpu(k, v)
     p = gpu_prefix(store, nq, gpu)
