@@ -67,25 +67,20 @@ __device__ __forceinline__ T pick(bool c, T x, T y) {
     return c ? x : y;
 }
 
-// 8 or 2 consecutive values at element `off` of an output of dtype DT
-template <int DT, int N, bool VEC>
-__device__ __forceinline__ void put_n(void *base, int64_t off, const float (&x)[N]) {
+// 8 consecutive values at element `off` of an output of dtype DT
+template <int DT, bool VEC>
+__device__ __forceinline__ void put8(void *base, int64_t off, const float (&x)[8]) {
     if constexpr (!VEC) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) ma_store_f(base, off + i, DT, x[i]);
+        for (int i = 0; i < 8; ++i) ma_store_f(base, off + i, DT, x[i]);
     } else if constexpr (DT == MA_F32) {
-        typedef __attribute__((ext_vector_type(N < 4 ? N : 4))) float fv;
+        typedef __attribute__((ext_vector_type(4))) float f32x4;
 #pragma unroll
-        for (int i = 0; i < N; i += 4) {
-            fv v;
-#pragma unroll
-            for (int e = 0; e < (N < 4 ? N : 4); ++e) v[e] = x[i + e];
-            *(fv *)((float *)base + off + i) = v;
-        }
+        for (int i = 0; i < 8; i += 4) *(f32x4 *)((float *)base + off + i) = f32x4{x[i], x[i + 1], x[i + 2], x[i + 3]};
     } else {
-        uint32_t w[N / 2];
+        uint32_t w[4];
 #pragma unroll
-        for (int i = 0; i < N / 2; ++i) {
+        for (int i = 0; i < 4; ++i) {
             if constexpr (DT == MA_BF16) {
                 w[i] = ma_pack_bf16x2(x[2 * i], x[2 * i + 1]);
             } else {
@@ -93,8 +88,7 @@ __device__ __forceinline__ void put_n(void *base, int64_t off, const float (&x)[
                        ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x[2 * i + 1]) << 16);
             }
         }
-        if constexpr (N == 2) *(uint32_t *)((uint16_t *)base + off) = w[0];
-        else *(uint4 *)((uint16_t *)base + off) = uint4{w[0], w[1], w[2], w[3]};
+        *(uint4 *)((uint16_t *)base + off) = uint4{w[0], w[1], w[2], w[3]};
     }
 }
 
@@ -130,7 +124,7 @@ __device__ __forceinline__ void dequant_tile(const PrefixArgs &a, int b, int h, 
 #pragma unroll
                 for (int c = 0; c < 8; ++c)
                     x[c] = ma_dq((w[c] >> (tr * 4)) & 15u, ma_f16_to_f32(sc[c]), ma_f16_to_f32(zp[c]));
-                put_n<DT, 8, VEC>(out, og + tr * on, x);
+                put8<DT, VEC>(out, og + tr * on, x);
             }
         }
     } else {
@@ -155,7 +149,7 @@ __device__ __forceinline__ void dequant_tile(const PrefixArgs &a, int b, int h, 
 #pragma unroll
                 for (int c = 0; c < 8; ++c)
                     x[c] = ma_dq((w[u] >> (4 * c)) & 15u, ma_f16_to_f32(sc[u]), ma_f16_to_f32(zp[u]));
-                if (j < q1) put_n<DT, 8, VEC>(out, ob + (int64_t)j * on + oct * 8, x);
+                if (j < q1) put8<DT, VEC>(out, ob + (int64_t)j * on + oct * 8, x);
             }
         }
     }
@@ -169,7 +163,7 @@ __device__ __forceinline__ void dequant_tile(const PrefixArgs &a, int b, int h, 
         float x[8];
 #pragma unroll
         for (int c = 0; c < 8; ++c) x[c] = ma_load_f(src, so + c, a.fdtype);
-        put_n<DT, 8, VEC>(out, ob + (int64_t)j * on + oct * 8, x);
+        put8<DT, VEC>(out, ob + (int64_t)j * on + oct * 8, x);
     }
 }
 
