@@ -324,8 +324,9 @@ __global__ void __launch_bounds__(VS_NT) vs_partial_bf_kernel(VsArgs a) {
 // at most 12 roundings of 2^-23 (v_dot2 may truncate), half of that in the root, and an ulp
 // for v_sqrt: under 16 f32 ulps of the true root.  Unless the root lies within VS_NEAR ulps of
 // the middle between two bf16 values, its rounding to bf16 is therefore the f64 one's; the
-// others (about 1 entry in 500), and sums outside [1e-30, 1e30] (no f32 product of theirs has
-// under- or overflowed), are done again in f64.
+// others (about 1 entry in 500), and sums outside [1e-30, 1e30], are done again in f64: within,
+// no product has overflowed, and those that have underflowed (at most 128, each below 2^-126)
+// would have added 1.5e-6 of the sum, 13 ulps of the root at most.
 constexpr int VS_NEAR = 64;
 template <bool SLOTS, bool HASQ, bool HASF>
 __global__ void __launch_bounds__(VS_NT) vs_score_bf_kernel(VsArgs a) {

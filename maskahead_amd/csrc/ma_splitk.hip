@@ -484,8 +484,10 @@ __device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, 
 
 // The kernel's arguments, loaded where they are asked for: behind an address the compiler cannot
 // follow back.  A short segment's loads, hoisted to the top of the kernel with all others, kept
-// two lane descriptors and the whole argument struct in scalar registers at once (94 to 113 of
-// them spilled to vector lanes in the D 128 kernels, 121 and 104 at D 64; none so).
+// two lane descriptors and the whole argument struct in scalar registers at once, and spilled 96
+// (masked 112) of them to vector lanes at D 128, 112 at D 64; so, none.  8 masked layers of
+// 6 997 tokens 443 -> 433 us, 8 of 32 800 637 -> 626.  (make_lane in each branch alone: 151 to
+// 172 spilled.)
 __device__ __forceinline__ const FwdArgs &args_again() {
     typedef __attribute__((address_space(4))) const FwdArgs *kernarg;
     uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();   // (the first parameter)
@@ -941,11 +943,13 @@ __global__ void __launch_bounds__(128) splitk_combine_kernel(FwdArgs a, ma_tenso
     }
 }
 
-// Pass 2 for at most CMB_FEW splits and many rows (a prefill chunk: 3 584 rows of 4 splits).
-// splitk_combine_kernel spends a 128-thread workgroup and two barriers on each row; here a
-// thread merges 8 channels of a row over all of its splits by itself, 16 rows of D 128 to a
-// workgroup, every load in flight at once and no barrier.  Bound by bytes: 14 336 rows, 38 MB,
-// 34.3 us a workgroup per row, 8.1 so.
+// Pass 2 for at most CMB_FEW splits, any count of rows.  splitk_combine_kernel spends a
+// 128-thread workgroup and two barriers on each row; here a thread merges 8 channels of a row
+// over all of its splits by itself, 16 rows of D 128 to a workgroup, every load in flight at
+// once and no barrier.  Bound by bytes for the many rows of a prefill chunk (14 336 of 4 splits,
+// 38 MB: 34.3 us a workgroup per row, 8.1 so), by its loads' latency for few, and still the
+// faster: launches of one graph, 7 rows of 2 splits 3.6 -> 2.9 us, 224 of 8 3.8 -> 3.4, 896 of 8
+// 4.4 -> 3.5, 3 584 of 8 10.5 -> 3.7.
 constexpr int CMB_FEW = 8, CMB_NT = 256;
 template <int D>
 __global__ void __launch_bounds__(CMB_NT) splitk_combine_few_kernel(FwdArgs a, ma_tensor4 out, float *mp_out,
@@ -1064,10 +1068,11 @@ int64_t partial_bytes(int BH, int slots, int R, int D) {
 // stages otherwise); as many splits as one dispatch wave holds, with or without the other
 // workgroups.  (Two waves of half the splits cost their first loads twice: 9 000 x 64, 84 row
 // tiles, 218 us for 182.)  The first, 7 row tiles with everything in the wave, stays unless
-// another is estimated to be faster by a twentieth.  A prefill chunk of 512 tokens, two layers,
-// before (7 row tiles, room for one short segment a row group) and now: 28 heads of 128 over 4
-// x 16 384 packed 528 -> 460 us (14 groups in 4 splits for 16 in 3), 32 heads over 8 x 14 000
-// 612 -> 541, 32 heads of 64 over 8 x 10 000 packed 342 -> 279.  Short prefixes (a sub-step's
+// another is estimated to be faster by a twentieth.  Two layers of a prefill chunk of 512 tokens,
+// whole, before (7 row tiles, room for one short segment a row group) and so, runs in turn: 28
+// heads of 128 over 4 x 16 384 packed 510 -> 441 us (14 groups in 4 splits for 16 in 3), 32
+// heads over 8 x 14 000 593 -> 522, 32 heads of 64 over 8 x 10 000 packed 342 -> 308, 28 of 64
+// over 4 x 9 000, 384 tokens, 180 -> 165; 32 over 8 x 3 000 packed, unchanged, 188 and 189.  Short prefixes (a sub-step's
 // 2 048 selected entries) spread over many CUs: each workgroup's cost is mostly fixed latency,
 // so more, shorter splits finish sooner (22.1 -> 17.9 us per sub-step at 4 KV heads x 2 048).
 constexpr int XCDS = 8;
