@@ -302,7 +302,7 @@ struct TwoSrc {
     int na;
 };
 
-// One append (or one quantizer call) in one launch.  kv 0 = keys, 1 = values; a workgroup
+// One append in one launch.  kv 0 = keys, 1 = values; a workgroup
 // belongs to one (lane, kv) and is one of
 //   head  the residual rows and, before a barrier, the key groups (the first gh) that read
 //         what these replace: in place, so one workgroup does both
@@ -327,7 +327,7 @@ struct AppendArgs {
     int64_t sq[2][4];
     _Float16 *s[2], *z[2];
     int64_t ss[2][3];
-    int H, D, lanes, kv0, nkv;   // kv kinds kv0 .. kv0 + nkv - 1
+    int H, D, lanes;
     int ntok;                    // tokens quantized
     int keep, first;             // residual rows [first, keep) written from source rows r + ntok
     int gh, nhead, nbulk;        // head groups; head (0 or 1) and bulk workgroups per (lane, kv)
@@ -526,9 +526,9 @@ struct ResidualPass {
 
 template <int DT, bool VEC>
 __global__ void __launch_bounds__(AP_NT) append_packed_kernel(AppendArgs A) {
-    const int units = A.lanes * A.nkv;
+    const int units = A.lanes * 2;
     const int u = blockIdx.x / units, y = blockIdx.x % units;
-    const int kv = A.kv0 + y / A.lanes, bh = y % A.lanes, b = bh / A.H, h = bh % A.H;
+    const int kv = y / A.lanes, bh = y % A.lanes, b = bh / A.H, h = bh % A.H;
     const RowSrc R = row_src<DT>(A.src[kv], b, h);
     ResidualPass<DT, VEC> pass;
     if (u < A.nhead) {
@@ -561,7 +561,7 @@ __global__ void __launch_bounds__(AP_NT) append_packed_kernel(AppendArgs A) {
 // Fills in the workgroups of an append of ntok quantized tokens and residual rows
 // [first, keep), and launches it (D divides 256 and is a multiple of 32).
 int launch_append(AppendArgs &A, int dtype, hipStream_t st, const char *who) {
-    const int na = A.src[A.kv0].na;
+    const int na = A.src[0].na;
     // the residual replaces rows that are read: those of quantized groups below row `keep`, and
     // its own (rows of `a` from `keep` on are written by nobody)
     const bool in_place = A.ntok > 0 && na > 0 && A.keep > 0;
@@ -569,11 +569,11 @@ int launch_append(AppendArgs &A, int dtype, hipStream_t st, const char *who) {
     A.nhead = in_place ? 1 : 0;
     A.nbulk = (A.ntok - A.gh * KG + BULK - 1) / BULK;
     const int ncopy = in_place ? 0 : std::max(0, (A.keep - A.first + COPY - 1) / COPY);
-    const int64_t wgs = (int64_t)(A.nhead + A.nbulk + ncopy) * A.lanes * A.nkv;
+    const int64_t wgs = (int64_t)(A.nhead + A.nbulk + ncopy) * A.lanes * 2;
     if (wgs == 0) return MA_OK;
     // 16-byte loads and stores: aligned bases and rows of whole 16-byte pieces
     bool vec = true;
-    for (int kv = A.kv0; kv < A.kv0 + A.nkv; ++kv) {
+    for (int kv = 0; kv < 2; ++kv) {
         const ma_tensor4 *ts[2] = {&A.src[kv].a, &A.src[kv].b};
         for (const ma_tensor4 *t : ts) {
             const int64_t m = dtype == MA_F32 ? 4 : 8;
@@ -593,15 +593,20 @@ int launch_append(AppendArgs &A, int dtype, hipStream_t st, const char *who) {
     return ma_check_launch(who);
 }
 
-// ---- quantizers of head dims that do not divide 256
+// ---- the quantizers alone (append_packed_kernel serves appends).  Bound by latency up to a few
+// thousand tokens: 4 heads of D 128 x 8 192, keys 5.1 us and values 5.1 (7.2 and 6.8 as a launch
+// of that kernel, whose workgroups are fewer and hold a residual pass's registers); 512 tokens
+// 4.6 and 4.2 (6.6 and 6.4), 32 768 12.0 and 12.0 (14.5 and 15.6), D 256 x 512 5.0 and 4.0 (10.0
+// and 9.8).
 // DT: the dtype, a compile-time constant so that a thread's loads are straight-line code
 // (all of them in flight at once) instead of one branch per element
-// keys: grid (T/KG, B*H), D threads; thread = one channel of one token group.
+// keys: a workgroup of D threads a token group; thread = one channel of it.
 template <int DT>
-__global__ void quantize_keys_kernel(ma_tensor4 src, int H, int D, uint8_t *kq, int64_t q0, int64_t q1, int64_t q2,
-                                     int64_t q3, _Float16 *ks, _Float16 *kz, int64_t s0, int64_t s1, int64_t s2) {
-    const int bh = blockIdx.y, b = bh / H, h = bh % H;
-    const int g = blockIdx.x;
+__global__ void quantize_keys_kernel(ma_tensor4 src, int ng, int H, int D, uint8_t *kq, int64_t q0, int64_t q1,
+                                     int64_t q2, int64_t q3, _Float16 *ks, _Float16 *kz, int64_t s0, int64_t s1,
+                                     int64_t s2) {
+    const int bh = blockIdx.x / ng, b = bh / H, h = bh % H;
+    const int g = blockIdx.x % ng;
     const int d = threadIdx.x;
     if (d >= D) return;
     float x[KG];
@@ -793,24 +798,10 @@ extern "C" int ma_quantize_keys(ma_tensor4 src, int B, int H, int T, int D, int 
         return MA_EINVAL;
     }
     if (T == 0) return MA_OK;
-    if (append_dim(D)) {
-        AppendArgs A{};
-        A.src[0] = TwoSrc{src, src, 0};
-        A.q[0] = (uint8_t *)kq;
-        A.s[0] = (_Float16 *)ks;
-        A.z[0] = (_Float16 *)kz;
-        std::copy(skq, skq + 4, A.sq[0]);
-        std::copy(sks, sks + 3, A.ss[0]);
-        A.H = H;
-        A.D = D;
-        A.lanes = B * H;
-        A.nkv = 1;
-        A.ntok = T;
-        return launch_append(A, src.dtype, (hipStream_t)stream, "ma_quantize_keys");
-    }
-    dim3 grid(T / KG, B * H);
+    const int ng = T / KG;
+    const dim3 grid((unsigned)((int64_t)ng * B * H));
 #define MA_QK(DT_)                                                                                                    \
-    hipLaunchKernelGGL(quantize_keys_kernel<DT_>, grid, dim3(D), 0, (hipStream_t)stream, src, H, D, (uint8_t *)kq,    \
+    hipLaunchKernelGGL(quantize_keys_kernel<DT_>, grid, dim3(D), 0, (hipStream_t)stream, src, ng, H, D, (uint8_t *)kq, \
                        skq[0], skq[1], skq[2], skq[3], (_Float16 *)ks, (_Float16 *)kz, sks[0], sks[1], sks[2])
     if (src.dtype == MA_BF16) MA_QK(MA_BF16);
     else if (src.dtype == MA_F16) MA_QK(MA_F16);
@@ -831,22 +822,6 @@ extern "C" int ma_quantize_values(ma_tensor4 src, int B, int H, int T, int D, in
         return MA_EINVAL;
     }
     if (T == 0) return MA_OK;
-    if (append_dim(D)) {
-        AppendArgs A{};
-        A.src[1] = TwoSrc{src, src, 0};
-        A.q[1] = (uint8_t *)vq;
-        A.s[1] = (_Float16 *)vs;
-        A.z[1] = (_Float16 *)vz;
-        std::copy(svq, svq + 4, A.sq[1]);
-        std::copy(svs, svs + 3, A.ss[1]);
-        A.H = H;
-        A.D = D;
-        A.lanes = B * H;
-        A.kv0 = 1;
-        A.nkv = 1;
-        A.ntok = T;
-        return launch_append(A, src.dtype, (hipStream_t)stream, "ma_quantize_values");
-    }
     int64_t items = (int64_t)B * H * T * (D / VG);
     int blocks = (int)((items + 255) / 256);
     if (blocks > 65535) blocks = 65535;
@@ -900,7 +875,6 @@ extern "C" int ma_append_packed(ma_tensor4 k_res, ma_tensor4 v_res, int old_res,
     A.H = H;
     A.D = D;
     A.lanes = B * H;
-    A.nkv = 2;
     A.ntok = move;
     A.keep = keep;
     A.first = move ? 0 : old_res;   // nothing quantized: the residual's rows stay, the new ones follow
