@@ -43,13 +43,16 @@ enum { SRC_PACKED = 0, SRC_DENSE = 1 };
 struct ScoreArgs {
     ma_tensor4 q;
     PrefixDev pre;
-    const int32_t *q_rows;   // NULL: the selection rows are block positions 0 .. T2 - 1
+    const int32_t *q_rows;   // NULL: the selection rows are block positions row0 .. row0 + T2 - 1
+    int row0;
     const float *mp, *lp;
     const void *op;  // prefix-only output [B*H, R, D] (op_dtype): the value centre's source
     int op_dtype;
     float *mass, *score;
     int H, G, T, T2, R, R2, row_tiles, value;
     int vround;    // 0, or MA_BF16 / MA_F16: packed values rounded to that dtype for the distance
+    int r2_total;  // selection rows of the whole call (the mean's divisor) when rows run in passes
+    int accum;     // this pass adds its share to mass (passes after the first; mass only)
     int nfast;     // whole tiles of the source kind per lane: tiles [0, nfast)
     int per;       // tiles per fast workgroup
     int fast_wgs;  // fast workgroups per lane (blockIdx.x below it); then one tail tile each
@@ -444,7 +447,7 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
     };
     // selection row rr = g * T2 + i: block position t (clamped into the block), row g * T + t
     auto sel_pos = [&](int rr, int g) {
-        return min(max(ident ? rr - g * T2 : sm.qr[rr - g * T2], 0), T - 1);
+        return min(max(ident ? a.row0 + rr - g * T2 : sm.qr[rr - g * T2], 0), T - 1);
     };
     const int rt_pad = 32 * row_tiles;
     // Q of the unit's row tile: in-order rows need no table, so their loads are issued
@@ -624,7 +627,7 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
         }
     };
 
-    const float inv_r2 = 1.0f / (float)R2;
+    const float inv_r2 = 1.0f / (float)a.r2_total;
     const int hist_rank = HIST ? a.hist_rank : 0;   // HIST: 1 or 2
     auto finish = [&](int tile, int rb, int db) {
         const int j = tile * TILE + lane;
@@ -643,14 +646,15 @@ __global__ void __launch_bounds__(NT) score_kernel(ScoreArgs a) {
             const int64_t o = (int64_t)bh * end + j;
             if (a.pre.mask) live = a.pre.mask[o] != 0;
             const float m = live ? s * inv_r2 : 0.f;
-            a.mass[o] = m;
+            const float mf = a.accum ? a.mass[o] + m : m;   // the mass after this pass
+            a.mass[o] = mf;
             float sc = 0.f;
             if (value) {
                 sc = live ? m * __builtin_sqrtf(sm.dist[db][lane]) : 0.f;
                 a.score[o] = sc;
             }
             // the key ma_topk_select gives this slot under the same mask
-            if constexpr (HIST) key = ma_order_key(live ? (hist_rank == 2 ? sc : m) : -__builtin_inff());
+            if constexpr (HIST) key = ma_order_key(live ? (hist_rank == 2 ? sc : mf) : -__builtin_inff());
         }
         if constexpr (HIST) {
             const int r = tile - tile0;   // tile of the run
@@ -1076,8 +1080,8 @@ __global__ void __launch_bounds__(SM_NT) score_small_kernel(ScoreArgs a, int uni
 // rows, Q in registers) over all of the workgroup's tokens: a K fragment read from LDS
 // serves two MFMAs, and the MFMAs of the next 32 tokens are issued between the exp2 of
 // these.  Bound by MFMA, VALU and exp2 issue, which add up.  (In passes of 512 rows, each a launch that staged
-// every tile again, a 512-token chunk of 7 heads over 16 384 tokens took 8 x 17.5 us, now 82; up to 512 rows score_kernel's
-// pipeline is the faster, 256 rows of 65 536 tokens of 8 heads 47 us to 79.)
+// every tile again, a 512-token chunk of 7 heads over 16 384 tokens took 8 x 17.5 us, now 82; up to
+// 512 rows, and in two passes of a long prefix, score_kernel's pipeline is the faster.)
 constexpr int MS_NT = 512, MS_WAVES = MS_NT / 64, MS_TILES = 7;
 
 template <int D>
@@ -1337,15 +1341,26 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
                                              ((uintptr_t)p->kf & 15) == 0 && ((uintptr_t)p->vf & 15) == 0 &&
                                              p->skf[0] % 16 == 0 && p->skf[1] % 16 == 0 && p->svf[0] % 16 == 0 &&
                                              p->svf[1] % 16 == 0);
-    const int row_tiles = (R2 + 31) / 32;
+    const int tiles = (n + TILE - 1) / TILE;
+    const bool packed = p->nq > 0;
+    // More rows than the 16 waves of score_kernel hold (mass only, checked above): two passes of
+    // it of equal size, the second adding to the first's mass, where two suffice and the prefix
+    // gives every CU 8 tiles, more than mass_rows_kernel keeps at once; else mass_rows_kernel.
+    // Passes and mass_rows_kernel, D 128: 518 rows over 4 x 65 536 16-bit tokens 60 us and 70,
+    // 896 77 and 89, 672 over 4 x 32 768 40.0 and 41.0, over 4 x 28 672 36.6 and 29.6; three
+    // passes of 1 120 rows over 4 x 65 536 105 and 101.  D 64, 672 over 4 x 65 536: packed 50.2
+    // and 51.7, 16-bit 55.0 and 50.5.
+    const bool many = R2 > MAX_R2;
+    const bool two = many && T2 <= 2 * (MAX_R2 / G) && (D == 128 || packed) && dense_vec_ok &&
+                     (int64_t)tiles * B * H >= 8 * ma_num_cus();
+    const int t2_pass = two ? (T2 + 1) / 2 : T2;
+    const int row_tiles = (G * t2_pass + 31) / 32;
     // one 1024-thread workgroup per CU: units of half a tile up to 8 row tiles, whole
     // tiles beyond.  (Two 512-thread workgroups per CU, NT = 512, measured 1.6x slower at
     // config 2: each workgroup loads its lane's Q and O_p rows in its prologue, so twice
     // the workgroups move twice those bytes.)
     const int halves = row_tiles <= 8 ? 1 : 2;
     const int wgs_per_cu = 1;
-    const int tiles = (n + TILE - 1) / TILE;
-    const bool packed = p->nq > 0;
     // whole tiles of the source kind go to the pipelined workgroups, the rest (a tile
     // straddling the packed / 16-bit boundary, 16-bit tail tiles, a partial last tile,
     // f32 or unaligned 16-bit prefixes) to one tail workgroup each
@@ -1364,6 +1379,7 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
     sa.q = q;
     sa.pre = prefix_dev(p, B, H);
     sa.q_rows = q_rows;
+    sa.r2_total = R2;
     sa.mp = mp;
     sa.lp = lp;
     sa.op = op;
@@ -1428,8 +1444,7 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
         // this pass does not build the histogram in-kernel: the select's own level-0 launch
         return ma_topk_level0_into_state(hist_rank == 2 ? score : mass, n, p->mask, n, B * H, n, topk_state, stream);
     }
-    // more rows than the 16 waves of score_kernel hold (mass only, checked above)
-    if (R2 > MAX_R2) {
+    if (many && !two) {
         // runs of at most MS_TILES tiles, as equal as whole dispatch waves allow
         const int all = (tiles * B * H + ma_num_cus() - 1) / ma_num_cus();
         const int waves = (all + MS_TILES - 1) / MS_TILES;
@@ -1458,16 +1473,24 @@ static int prefix_scores(const char *who, ma_tensor4 q, int B, int Hq, int T, in
         if (halves == 1) MA_SCORE(D_, S_, 1);     \
         else MA_SCORE(D_, S_, 2);                 \
     } while (0)
-    sa.hist_rank = hist_rank;
-    if (D == 128) {
-        if (packed) MA_SCORE_I(128, SRC_PACKED);
-        else MA_SCORE_I(128, SRC_DENSE);
-    } else {
-        if (packed) MA_SCORE_I(64, SRC_PACKED);
-        else MA_SCORE_I(64, SRC_DENSE);
+    for (int t0 = 0; t0 < T2; t0 += t2_pass) {
+        sa.q_rows = q_rows ? q_rows + t0 : nullptr;
+        sa.row0 = t0;
+        sa.T2 = min(t2_pass, T2 - t0);
+        sa.R2 = G * sa.T2;
+        sa.row_tiles = (sa.R2 + 31) / 32;
+        sa.accum = t0 > 0;
+        sa.hist_rank = t0 + t2_pass >= T2 ? hist_rank : 0;   // the last pass sees the final mass
+        if (D == 128) {
+            if (packed) MA_SCORE_I(128, SRC_PACKED);
+            else MA_SCORE_I(128, SRC_DENSE);
+        } else {
+            if (packed) MA_SCORE_I(64, SRC_PACKED);
+            else MA_SCORE_I(64, SRC_DENSE);
+        }
+        rc = ma_check_launch(who);
+        if (rc) return rc;
     }
-    rc = ma_check_launch(who);
-    if (rc) return rc;
 #undef MA_SCORE_I
 #undef MA_SCORE
     // lanes beyond 31-bit offsets run the kernel without the in-kernel histogram

@@ -5,6 +5,7 @@ every prefix kind, against the oracle from the same statistics."""
 import pytest
 import torch
 
+from maskahead_amd.kernels import prefix_scores_topk, topk_ascending
 from maskahead_amd.kernels.splitk import Prefix, prefix_scores, splitk_attention
 from oracle import attention as OA
 
@@ -57,3 +58,32 @@ def test_mass_of_many_rows(gpu, kind, n, heads, d, t, rows, masked):
     assert rel_err(mass, wmass) < 2e-5
     if masked:
         assert torch.all(mass.cpu()[mask == 0] == 0)
+
+
+@pytest.mark.parametrize("kind,rows", [("packed", None), ("packed", "some"), ("bf16", None)])
+def test_mass_of_many_rows_in_two_passes(gpu, kind, rows):
+    """516 to 524 selection rows over 8 x 16 500 tokens, at least 8 tiles a CU: two passes, the
+    second adding to the first's mass; the select's histogram is of the sum."""
+    hq, hkv, d, n, t = 32, 8, 128, 16500, 131
+    q, k, v, kc, vc = layer_inputs(hq=hq, hkv=hkv, d=d, n=n, t=t, seed=n, dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(n)
+    mask = (torch.rand((1, hkv, n), generator=g) > 0.3).to(torch.uint8)
+    mask[:, :, 0] = 1
+    if kind == "packed":
+        nq = (n - 32) // 32 * 32
+        store, nq = packed_cpu(k[:, :, :nq], v[:, :, :nq])
+        kd, _ = dequant_cpu(store, nq)
+        p = gpu_prefix(store, nq, gpu, kf=k[:, :, nq:], vf=v[:, :, nq:], mask=mask)
+        k_used = torch.cat([kd, k[:, :, nq:].float()], 2)
+    else:
+        k_used = k.float()
+        p = Prefix.dense(k.to(gpu), v.to(gpu), mask=mask.to(gpu))
+    qg = q.to(gpu)
+    _, stats = splitk_attention(qg, p, kc.to(gpu), vc.to(gpu), want_prefix=True)
+    mp, lp, op = (x.cpu() for x in stats[:3])
+    sel = list(range(t)) if rows is None else list(range(t - 1, 1, -1))
+    mass, _ = prefix_scores(qg, p, stats, sel, value=False)
+    want, _ = OA.prefix_scores(q, k_used, None, mp, lp, None, sel, mask=mask, value_aware=False)
+    assert rel_err(mass, want) < 2e-5 and torch.all(mass.cpu()[mask == 0] == 0)
+    m2, _, idx = prefix_scores_topk(qg, p, stats, sel, 500, value=False, rank="mass")
+    assert torch.equal(m2, mass) and torch.equal(idx, topk_ascending(mass, 500, p.mask))
