@@ -204,7 +204,8 @@ struct FwdSmem {
 // covers the wait: there the turn through LDS only cost (544 tokens 40.9 -> 41.5 us a step).
 // So it does for few row tiles, whose fragments' loads are few: sub-steps over 2 048 entries, 28
 // query heads over 4, direct and turned: 2 row tiles 11.11 and 11.44 us, 4 12.63 and 12.68, 5
-// 14.41 and 14.39, 7 15.76 and 15.25.
+// 14.41 and 14.39, 7 15.76 and 15.25.  (Both in one kernel, chosen there, slowed both: pass 1 over
+// 32 768 tokens 20.2 us at 2 row tiles, alone 19.8, at 7 27.7, alone 27.2.)
 constexpr int FEW_TILES = 4;
 template <int D>
 struct QRows {
@@ -495,10 +496,12 @@ __device__ __forceinline__ const FwdArgs &args_again() {
     return *(const FwdArgs *)(kernarg)p;
 }
 
-// MASK: the prefix has a slot mask (packed sources: their splits are whole 64-token tiles
-// either way, what is left goes to short_segment, so no tile needs bounds)
-template <int D, int SRC, bool MASK>
+// OPT, packed sources: MASK, the prefix has a slot mask (their splits are whole 64-token tiles
+// either way, what is left goes to short_segment, so no tile needs bounds); 16-bit sources: TURN,
+// query rows come through QRows.
+template <int D, int SRC, bool OPT>
 __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
+    constexpr bool MASK = SRC == 0 && OPT, TURN = SRC != 0 && OPT;
     __shared__ FwdSmem<D> S;
     using Shape = StageShape<KLANES, D, SRC == 0 ? ST_PACKED : ST_DENSE>;
     constexpr int NKS = D / 16;
@@ -734,7 +737,7 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
     // prologue: tiles 0 and 1 staged, tile 2's loads in flight; Q of the row tile
     if (nt > 0) load_tile(0);
     bf16x8_t qf[NKS];
-    if (SRC == 0 || nS <= FEW_TILES) {
+    if constexpr (!TURN) {
         if (is_s) {
             const int g = row_ok ? row / a.T : 0, t = row_ok ? row % a.T : 0;
             const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
@@ -1250,12 +1253,13 @@ int launch_partial_d(const Plan &pl, hipStream_t st) {
         fa.with_tail = 0;
         fa.with_cur = 1;
         const dim3 grid((nsf + 1) * units);
+        const bool turn = fa.group_tiles > FEW_TILES;
         const bool bf = (nf == 0 || fa.pre.fdtype == MA_BF16) &&
                         (fa.Tc == 0 || (fa.kc.dtype == MA_BF16 && fa.vc.dtype == MA_BF16));
-        if (bf)
-            hipLaunchKernelGGL((splitk_fwd_kernel<D, 2, true>), grid, dim3(NTH), 0, st, fa);
-        else
-            hipLaunchKernelGGL((splitk_fwd_kernel<D, 1, true>), grid, dim3(NTH), 0, st, fa);
+        if (bf && turn) hipLaunchKernelGGL((splitk_fwd_kernel<D, 2, true>), grid, dim3(NTH), 0, st, fa);
+        else if (bf) hipLaunchKernelGGL((splitk_fwd_kernel<D, 2, false>), grid, dim3(NTH), 0, st, fa);
+        else if (turn) hipLaunchKernelGGL((splitk_fwd_kernel<D, 1, true>), grid, dim3(NTH), 0, st, fa);
+        else hipLaunchKernelGGL((splitk_fwd_kernel<D, 1, false>), grid, dim3(NTH), 0, st, fa);
     }
     return ma_check_launch("ma_splitk_partial");
 }
