@@ -378,31 +378,29 @@ __device__ __forceinline__ void pv_regs(const uint16_t *Vt, const bf16x8_t *pb, 
             acc[dt] = ma_mfma32(*(const bf16x8_t *)&vrow[dt * 32 * VS + c * 16], pb[c], acc[dt]);
 }
 
-// A short segment of one (lane, row group) of the packed kernel, its tiles staged
-// synchronously by every thread, then S^T, softmax and PV:
-//   the current block (block-causal mask), partial to slot nsplit;
-//   the packed prefix's tail: what its whole 64-token tiles leave, an odd key group of 32
-//   tokens and the 16-bit residual, partial to the slot behind the splits.
-template <int D>
+// A short segment of one (lane, row group) of the packed kernel, its tiles staged by every
+// thread, then S^T, softmax and PV:
+//   CUR   the current block (block-causal mask), partial to slot nsplit;
+//   else  the packed prefix's tail: what its whole 64-token tiles leave, an odd key group of 32
+//         tokens and the 16-bit residual, partial to the slot behind the splits.
+// Beside splits of a tile or two it ends last, so a tile's loads, packed and 16-bit, are all
+// issued before the first is waited for.  (One code for both, its loads behind branches: pass 1
+// over 4 heads x 1 024 packed tokens 9.3 us, now 8.5, 8.0 without a current block; of D 64 6.9,
+// 6.3 and 5.8.)
+template <int D, bool CUR>
 __device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, const Lane &L, FwdSmem<D> &S) {
     constexpr int NKS = D / 16;
     constexpr int NDT = D / 32;
+    constexpr int CH = D / 8, NK = TILE * CH / NTH;        // 16-bit K items a thread; one of V at most
     const int bh = wk.bh, b = bh / a.H, h = bh % a.H;
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, c32 = lane & 31, hf = lane >> 5;
-    const bool cur = wk.cur;
-    Dense kc, vc;
-    if (cur) {
-        kc = dense_lane(a.kc.ptr, a.kc.s, a.kc.dtype, b, h);
-        vc = dense_lane(a.vc.ptr, a.vc.s, a.vc.dtype, b, h);
-    } else {
-        kc = Dense{L.kf, L.kf_n, L.fdtype, L.esz};
-        vc = Dense{L.vf, L.vf_n, L.fdtype, L.esz};
-    }
-    const int beg = cur ? 0 : a.tok_end;                   // first token of the segment
-    const int ntok = cur ? a.Tc : a.tail_end - beg;
-    const int np = cur ? 0 : L.nq - beg;                   // its packed tokens: 0 or one group
-    const uint8_t *mask = cur ? nullptr : L.mask;
+    const Dense kc = CUR ? dense_lane(a.kc.ptr, a.kc.s, a.kc.dtype, b, h) : Dense{L.kf, L.kf_n, L.fdtype, L.esz};
+    const Dense vc = CUR ? dense_lane(a.vc.ptr, a.vc.s, a.vc.dtype, b, h) : Dense{L.vf, L.vf_n, L.fdtype, L.esz};
+    const int beg = CUR ? 0 : a.tok_end;                   // first token of the segment
+    const int ntok = CUR ? a.Tc : a.tail_end - beg;
+    const int np = CUR ? 0 : L.nq - beg;                   // its packed tokens: 0 or one group
+    const uint8_t *mask = CUR || !L.mask ? nullptr : L.mask + beg;
     const int nt = (ntok + TILE - 1) / TILE;
     const int nS = min(a.group_tiles, a.row_tiles - wk.rg * a.group_tiles);
     const bool is_s = wave < nS;
@@ -410,14 +408,12 @@ __device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, 
     const int row = rtile * 32 + c32;
     const bool row_ok = row < a.R;
     const int qpos = a.q_pos0 + (row_ok ? row % a.T : 0);
-    const bool causal = cur && a.causal > 0;
+    const bool causal = CUR && a.causal > 0;
     bf16x8_t qf[NKS];
     if (is_s) {
         const int g = row_ok ? row / a.T : 0, t = row_ok ? row % a.T : 0;
         const int64_t qb = b * a.q.s[0] + (int64_t)(h * a.G + g) * a.q.s[1] + (int64_t)t * a.q.s[2];
         ma_load8n_as_bf16<NKS>(a.q.ptr, a.q.dtype, [&](int ks) { return qb + ks * 16 + hf * 8; }, qf);
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) qf[ks] = row_ok ? qf[ks] : bf16x8_t{};
     }
     float m_ref = -INFINITY, m_true = -INFINITY, l = 0.f;
     f32x16_t acc[NDT];
@@ -426,42 +422,51 @@ __device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, 
     for (int i = 0; i < nt; ++i) {
         const int n0 = i * TILE;
         const int valid = ntok - n0;
-        const int pk = i == 0 ? np : 0;                    // packed tokens of this tile
-        uint32_t w[8];
+        const int pk = !CUR && i == 0 ? np : 0;            // packed tokens of this tile
+        // the packed group: thread u < D its K item u (key group 0 of the tile), then the V items
+        const int pu = tid - D;
+        const bool pk_k = tid < D, pk_v = pu >= 0 && pu < 2 * D && (pu & 31) < KGRP / 2;
+        uint32_t wp[8], wk16[NK][8], wv16[8];
         if (pk) {
-            for (int u = tid; u < D; u += NTH) {           // the items of key group 0 of the tile
-                load_k_packed<D>(w, L, u, beg, L.nq);
-                store_k_packed<D>(S.u.t.kt[0].k, w, u);
-            }
-            for (int u = tid; u < 2 * D; u += NTH) {
-                if ((u & 31) >= KGRP / 2) continue;        // token pairs of the group
-                uint32_t fl;
-                load_v_packed<D>(w, fl, L, u, beg, L.nq);
-                store_v_packed<D>(S.u.t.vt[0].vt, w, u);
-            }
+            uint32_t fl;
+            if (pk_k) load_k_packed<D>(wp, L, tid, beg, L.nq);
+            else if (pk_v) load_v_packed<D>(wp, fl, L, pu, beg, L.nq);
         }
-        // 16-bit tokens [pk, valid) of the tile; tokens from `valid` on are staged as zeros
+        // 16-bit tokens [pk, valid) of the tile (items outside repeat the nearest's loads);
+        // tokens from `valid` on are staged as zeros
+        const bool any = CUR || valid > pk;
         const int64_t r0 = n0 - np;                        // row of the tile's first token
-        const char *kb = kc.base + r0 * kc.sn * kc.esz;
-        for (int u = tid; u < TILE * D / 8; u += NTH) {
-            const int t = u / (D / 8);
-            if (t < pk) continue;
-            const bool ok = t < valid;
-            if (ok) load_k_dense<D>(w, kb, kc.sn, kc.dtype, kc.esz, u, valid);
-            store_k_dense<D>(S.u.t.kt[0].k, w, u, kc.dtype, ok);
+        const char *kb = kc.base + r0 * kc.sn * kc.esz, *vb = vc.base + r0 * vc.sn * vc.esz;
+        const int vt = 2 * (tid % (TILE / 2)), vch = tid / (TILE / 2);   // V: token pair, 8 channels
+        if (any) {
+#pragma unroll
+            for (int e = 0; e < NK; ++e) {
+                const int u = tid + e * NTH;
+                load_k_dense<D>(wk16[e], kb, kc.sn, kc.dtype, kc.esz, max(u / CH, pk) * CH + u % CH, valid);
+            }
+            if (vch < CH)
+                load_v_dense<D>(wv16, vb, vc.sn, vc.dtype, vc.esz, vch * (TILE / 2) + max(vt, pk) / 2, valid);
         }
-        const char *vb = vc.base + r0 * vc.sn * vc.esz;
-        for (int u = tid; u < TILE / 2 * D / 8; u += NTH) {
-            const int t = 2 * (u % (TILE / 2));
-            if (t < pk) continue;
-            const bool l0 = t < valid && (!mask || mask[beg + n0 + t]);
-            const bool l1 = t + 1 < valid && (!mask || mask[beg + n0 + t + 1]);
-            if (t < valid) load_v_dense<D>(w, vb, vc.sn, vc.dtype, vc.esz, u, valid);
-            store_v_dense<D>(S.u.t.vt[0].vt, w, u, vc.dtype, l0, l1);
+        const bool live = lane < valid && (!mask || mask[n0 + min(lane, valid - 1)]);
+        const bool l0 = vt < valid && (!mask || mask[n0 + min(vt, valid - 1)]);
+        const bool l1 = vt + 1 < valid && (!mask || mask[n0 + min(vt + 1, valid - 1)]);
+        if (pk) {
+            if (pk_k) store_k_packed<D>(S.u.t.kt[0].k, wp, tid);
+            else if (pk_v) store_v_packed<D>(S.u.t.vt[0].vt, wp, pu);
         }
+#pragma unroll
+        for (int e = 0; e < NK; ++e) {
+            const int u = tid + e * NTH, t = u / CH;
+            if (t >= pk) store_k_dense<D>(S.u.t.kt[0].k, wk16[e], u, kc.dtype, t < valid);
+        }
+        if (vch < CH && vt >= pk) store_v_dense<D>(S.u.t.vt[0].vt, wv16, vch * (TILE / 2) + vt / 2, vc.dtype, l0, l1);
         if (wave == 0) {
-            const uint64_t m = __ballot(lane < valid && (!mask || mask[beg + n0 + min(lane, valid - 1)]));
+            const uint64_t m = __ballot(live);
             if (lane == 0) S.kmask[0] = m;
+        }
+        if (i == 0 && is_s) {
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) qf[ks] = row_ok ? qf[ks] : bf16x8_t{};
         }
         __syncthreads();  // tile staged
         if (is_s) {
@@ -479,7 +484,7 @@ __device__ __forceinline__ void short_segment(const FwdArgs &a, const Work &wk, 
         __syncthreads();  // buffers free
     }
     if (is_s)
-        write_partial<D>(a, acc, m_ref, m_true, l, bh, cur ? a.nsplit : a.slot0 + a.nsp, rtile, c32, hf, lane,
+        write_partial<D>(a, acc, m_ref, m_true, l, bh, CUR ? a.nsplit : a.slot0 + a.nsp, rtile, c32, hf, lane,
                          &S.u.o[wave][0]);
 }
 
@@ -515,7 +520,8 @@ __global__ void __launch_bounds__(NTH) splitk_fwd_kernel(FwdArgs a) {
     if constexpr (SRC == 0) {
         if (wk.seg != SEG_SPLIT) {
             const FwdArgs &args = args_again();
-            short_segment<D>(args, wk, make_lane(args.pre, b, h, bh), S);
+            if (wk.seg == SEG_CUR) short_segment<D, true>(args, wk, Lane{}, S);
+            else short_segment<D, false>(args, wk, make_lane(args.pre, b, h, bh), S);
             return;
         }
     }
