@@ -202,11 +202,12 @@ struct FwdSmem {
 // tile the last of them came ~2 000 cycles after the tile itself (8 000): a sub-step over
 // 2 048 entries 16.4 -> 15.9 us.  A packed tile is a third of that and its dequantization
 // covers the wait: there the turn through LDS only cost (544 tokens 40.9 -> 41.5 us a step).
-// So it does for few row tiles, whose fragments' loads are few: sub-steps over 2 048 entries, 28
-// query heads over 4, direct and turned: 2 row tiles 11.11 and 11.44 us, 4 12.63 and 12.68, 5
-// 14.41 and 14.39, 7 15.76 and 15.25.  (Both in one kernel, chosen there, slowed both: pass 1 over
-// 32 768 tokens 20.2 us at 2 row tiles, alone 19.8, at 7 27.7, alone 27.2.)
-constexpr int FEW_TILES = 4;
+// So it does for few row tiles, whose fragments' loads are few.  Pass 1 of 28 query heads over 4,
+// direct and turned: 2 row tiles over 2 048 entries 6.1 and 6.4 us, over 32 768 19.8 and 20.2; 3
+// 6.7 and 6.8, 20.4 and 20.6 (over 8 192 10.2 and 9.9); 4 7.1 and 7.1, 21.0 and 21.0, over 8 192
+// 10.6 and 10.1, of D 64 over 32 768 14.6 and 14.3; 7 over 32 768 28.4 and 27.2.  (Both in one
+// kernel, chosen there, slowed both: 20.2 us at 2 row tiles, 27.7 at 7.)
+constexpr int FEW_TILES = 3;
 template <int D>
 struct QRows {
     static constexpr int CH = D / 8, NI = 32 * CH / 64;
