@@ -1,6 +1,6 @@
 """Benchmark of the MI355X read path: step 0 of a sparse layer at the headline shape.
 
-Workload: packed int4 k4v4 cache, prefix 32768 tokens, batch
+Workload (the headline shape): packed int4 k4v4 cache, prefix 32768 tokens, batch
 1, 28 query / 4 KV heads, head_dim 128, mask block of 32 queries (all 32 are selection
 rows), read budget 2048 per KV head.  One layer step = split-K attention over
 [prefix | block] with prefix statistics, the value-aware score pass, the read-set top-k

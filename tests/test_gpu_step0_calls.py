@@ -78,3 +78,27 @@ def test_rows_changed_in_place(gpu, dtype, rows, where):
         got = _step0(bufs, layer, rows)
         want = _step0(Step0Buffers(), layer, list(values))
         assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3]) and torch.equal(got[4], want[4])
+
+
+def test_captured_f16_step0(gpu):
+    """A captured f16 step 0 owns its copy: replays over new queries, with eager calls of the same
+    prefix between them, equal the eager results."""
+    q, kc, vc, p = _layer(gpu, 6)
+    static = [x.clone() for x in (q, kc, vc)]
+    bufs, ws, eager = Step0Buffers(), Step0Buffers(), Step0Buffers()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _step0(bufs, (*static, p), workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out, stats, mass, score, idx = _step0(bufs, (*static, p), workspace=ws)
+    for scale in (1.0, 0.5, -0.75, 1.25):
+        for s, x in zip(static, (q, kc, vc)):
+            s.copy_(x * scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = _step0(eager, (*static, p))
+        assert torch.equal(out, want[0]) and torch.equal(mass, want[2]) and torch.equal(score, want[3])
+        assert torch.equal(idx, want[4]) and torch.equal(stats[3].kf, want[1][3].kf)
